@@ -1248,6 +1248,7 @@ int run_gemv_matrix(nx_ctx *c, int fmt, const RolePlane &pl, const float *x, int
 }  // namespace
 
 int launch_gemv_matrix(nx_ctx *c, int fmt, const RolePlane &pl, const float *x, int T, float *out) {
+  if (mfd_takes(fmt, pl, x, T)) return launch_mfd(c, fmt, pl, x, T, out);
   return run_gemv_matrix(c, fmt, pl, x, T, out);
 }
 bool gemv_row_fits(int fmt, int nseg) {

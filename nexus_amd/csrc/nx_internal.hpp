@@ -296,6 +296,9 @@ int launch_gemv_gateup(nx_ctx *c, const GemvPlan &p);
 // out[t][r] = sum_c W[r][c] x[t][c] for one resident matrix (x rows pl.cols
 // floats apart, out rows pl.rows floats apart)
 int launch_gemv_matrix(nx_ctx *c, int fmt, const RolePlane &pl, const float *x, int T, float *out);
+// the same on MFMA for several tokens (nx_mfd.hip); mfd_takes: the calls it takes
+bool mfd_takes(int fmt, const RolePlane &pl, const float *x, int T);
+int launch_mfd(nx_ctx *c, int fmt, const RolePlane &pl, const float *x, int T, float *out);
 // whether a row of nseg segments fits the register-resident GEMV
 bool gemv_row_fits(int fmt, int nseg);
 int launch_gemv_down(nx_ctx *c, const GemvPlan &p);
