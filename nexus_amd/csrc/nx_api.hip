@@ -965,6 +965,18 @@ int nx::moe_forward(nx_ctx *c, const nx_experts *ex, const float *d_x, const flo
     const double kk = std::min(1.0, (double)k / E);
     const double act = std::max(1.0, E * (1.0 - std::pow(1.0 - kk, (double)T)));
     const double tpe = (double)T * k / act;
+    // The split path streams the active experts' weights at 4.3 TB/s behind
+    // about 35 us of launches, so it wins over wider ranges where an expert is
+    // large: `large` from 7 M weights a matrix (measured at 4096 x 1792 and up).
+    // In the fixed scratch array of nx_moe_forward_noalloc a batch that its
+    // workspace would not fit keeps the narrower ranges, whose other paths
+    // need less.
+    const bool fits = !c->scratch_mode ||
+                      mfv_bytes(ex, T, k) + (size_t)T * k * 64 + (size_t)E * 64 + (1u << 20) <= kScratchBytes;
+    const double weights = (double)H * ex->F;
+    const bool large = fits && weights >= 7e6;
+    const bool q8 = ex->fmt == NX_FMT_Q8_0;
+    const bool split_fmt = ex->fmt == NX_FMT_Q4_K || ((ex->fmt == NX_FMT_Q4_0 || q8) && mfv_supports(ex));
     if (ex->fmt == NX_FMT_Q2_K) {
       // The GEMV or the split-activation path (Q2_K has no grouped GEMM).
       // Measured (ms, GEMV / split): Mixtral 2 tokens 0.101 / 0.122, 4:
@@ -977,40 +989,38 @@ int nx::moe_forward(nx_ctx *c, const nx_experts *ex, const float *d_x, const flo
       else
         use = (tpe >= 1.8 || ((long)T * k >= 64 && tpe >= 1.2)) ? NX_PATH_MFMA_SPLIT
                                                                  : NX_PATH_GEMV;
-    } else if (ex->fmt == NX_FMT_Q4_K && shared && ex->Fs == ex->F) {
+    } else if (split_fmt && shared && ex->Fs == ex->F && (large || ex->fmt == NX_FMT_Q4_K)) {
       // A shared expert sees every token: the GEMV walks it a token pair at
       // a time, the split-activation path 16 tokens at a time.  Measured
-      // (DeepSeek shapes, ms, GEMV / split / grouped GEMM): 2 tokens 0.115 /
-      // 0.173 / 0.268, 4: 0.270 / 0.264 / 0.321, 8: 0.887 / 0.508 / 0.588,
-      // 16: 3.69 / 0.904 / 0.996, 32: - / 1.31 / 1.52, 64: - / 1.76 / 2.04;
-      // the grouped GEMM (64-pair tiles at these counts) from the routed
-      // experts' 8 tokens each: 192 tokens (6 each) split 2.08-2.18 / GEMM
-      // 2.11, 256 tokens (8 each) 2.19-2.29 / 2.13.
-      if (tpe >= 8.0)
+      // (DeepSeek shapes, us, GEMV / split / grouped GEMM): Q4_K 2 tokens 105
+      // / 128 / 233, 4: 265 / 196 / 282, 27: 9257 / 836 / 1251, 128: - / 1546 /
+      // 1989, 256 (8 per routed expert): - / 1836 / 2090, 400 (12.5): - / 2105
+      // / 2123; Q4_0 4: 232 / 198 / 281, 27: - / 950 / 1226, 128: - / 1665 /
+      // 1960; Q8_0 8: 840 / 542 / 643, 27: - / 1357
+      // / 1524, 300 (9.4): - / 2924 / 2730.
+      if (tpe >= (large && !q8 ? 12.0 : 8.0))
         use = NX_PATH_MFMA_BF16;
       else
-        use = T >= 4 ? NX_PATH_MFMA_SPLIT : NX_PATH_GEMV;
-    } else if ((ex->fmt == NX_FMT_Q4_K ||
-                ((ex->fmt == NX_FMT_Q4_0 || ex->fmt == NX_FMT_Q8_0) && mfv_supports(ex))) &&
-               !shared) {
-      // Measured crossovers (Mixtral and Qwen3 shapes): the GEMV re-reads an
-      // expert's weights per pair of its tokens and wins below ~2 tokens per
-      // expert; the split-activation MFMA path reads them once per 16 tokens
-      // and wins up to ~12 (Mixtral: 0.31 against 0.36 ms at 8 tokens per
-      // expert, 0.45 against 0.36 at 16; Qwen3: 0.17 / 0.20 at 8, 0.24 /
-      // 0.21 at 16); the grouped GEMM beyond.  Q4_0 (ms, GEMV / split /
-      // grouped GEMM): Mixtral 2 tokens per expert 0.183 / 0.233 / 0.290,
-      // 4: 0.368 / 0.253 / 0.295, 8: - / 0.272 / 0.297, 16: - / 0.343 /
-      // 0.299; Qwen3 1.2: 0.079 / 0.069 / 0.095, 4: 0.285 / 0.135 / 0.160.
-      // Q8_0: Mixtral 2 tokens per expert 0.287 / 0.317 / 0.351, 4: 0.600 /
-      // 0.344 / 0.359, 8: - / 0.366 / 0.379, 16: - / 0.435 / 0.383; Qwen3
-      // 1.2: 0.083 / 0.081 / 0.103, 4: 0.347 / 0.169 / 0.184, 8: - / 0.175 /
-      // 0.188, 16: - / 0.247 / 0.192.  (With a shared expert Q4_0 and Q8_0
-      // keep the rule below: at DeepSeek's shape the split path and the
-      // grouped GEMM are within 4% from 16 tokens.)
-      if (tpe >= 12.0)
+        use = T >= (q8 ? 6 : 4) ? NX_PATH_MFMA_SPLIT : NX_PATH_GEMV;
+    } else if (split_fmt && !shared) {
+      // The GEMV re-reads an expert's weights per pair of its tokens, the
+      // split-activation path reads them once per 16 tokens, and the grouped
+      // GEMM once, at bf16 operands.  Measured (us, GEMV / split / grouped
+      // GEMM) by tokens per expert: Mixtral Q4_0 1.1: 80 / 96 / 176, 1.5: 154 /
+      // 130 / 240, 2.0: 249 / 155 / 244; Q4_K 1.3: 128 / 107 / 201, 2.2: 454 /
+      // 156 / 254, 8: 906 / 215 / 301, 12: - / 241 / 304, 16: - / 320 / 305;
+      // Q8_0 2.0: 320 / 239 / 295, 8: - / 338 / 363, 16: - / 540 / 365; Qwen3
+      // Q4_K 1.1: 45 / 50 / 68, 1.3: 107 / 64 / 93, 8: - / 132 / 151, 12.5: -
+      // / 137 / 153, 16: - / 155 / 156.  Smaller layers (GEMV / split): 8
+      // experts of 4096 x 1792 Q4_K 1.3: 38 / 37, 1.6: 57 / 43, Q8_0 1.6: 48 /
+      // 54, 2.2: 59 / 54; 1024 x 2048 Q4_K 1.3: 31 / 35, 1.6: 42 / 35; 512 x
+      // 1024 Q4_K 1.6: 25 / 34, 2.2: 35 / 36, 3.1: 46 / 37; 64 experts of 1024
+      // x 768, top 8, 1.1: 35 / 35, 1.3: 53 / 36.
+      const long pairs = (long)T * k;
+      if (tpe >= (large && !q8 ? 13.0 : 12.0))
         use = NX_PATH_MFMA_BF16;
-      else if (tpe >= 3.0 || ((long)T * k >= 64 && tpe >= 1.2))
+      else if (tpe >= 3.0 || (pairs >= 64 && tpe >= 1.2) || (fits && pairs >= 40 && tpe >= 1.25) ||
+               (large && tpe >= (q8 ? 2.0 : 1.28)) || (fits && !q8 && weights >= 2e6 && tpe >= 1.6))
         use = NX_PATH_MFMA_SPLIT;
       else
         use = NX_PATH_GEMV;
@@ -1067,16 +1077,23 @@ int nx::moe_forward(nx_ctx *c, const nx_experts *ex, const float *d_x, const flo
     const int max_tiles = mfv_max_tiles(T, k, E, shared);
     int32_t *d_tiles;
     NX_TRY(ws(c, WS_TILES, 2 + 2 * (size_t)max_tiles, &d_tiles));
+    // activation rows are read as float4 runs of whole chunks
+    if (reinterpret_cast<uintptr_t>(d_x) & 15)
+      return fail(NX_ERR_UNSUPPORTED, "the split-activation MFMA path needs 16-byte aligned inputs");
+    uint8_t *d_rec;
+    NX_TRY(mfv_records(c, ex, T, k, &d_rec));
+    SplitJob split{d_x, (size_t)T * H / 256, d_rec, ex->fmt, false};
     // (the fused router lists no shared-expert tiles)
     if (!shared && route_permute_fusable(T, E, k)) {
       NX_TRY(launch_route_permute(c, d_logits, T, E, k, score_mode, d_exp, d_w, d_cnt, d_ec, d_off,
-                                  d_pt, d_ps, d_inv, d_act, kMfvTileM, d_tiles, nullptr, 0));
+                                  d_pt, d_ps, d_inv, d_act, kMfvTileM, d_tiles, nullptr, 0, &split));
     } else {
       NX_TRY(launch_route(c, d_logits, T, E, k, score_mode, d_exp, d_w, d_cnt));
       NX_TRY(launch_permute(c, d_exp, d_cnt, T, k, E, kMfvTileM, d_ec, d_off, d_pt, d_ps, d_inv,
-                            d_act, d_tiles, shared ? T : 0));
+                            d_act, d_tiles, shared ? T : 0, 0, nullptr, &split));
     }
-    MfvPlan mp{ex, T, k, d_x, d_pt, d_off, d_tiles, max_tiles, d_w, d_cnt, d_inv, d_out, d_residual};
+    if (!split.done) NX_TRY(launch_mfv_split(c, split));
+    MfvPlan mp{ex, T, k, d_rec, d_pt, d_off, d_tiles, d_w, d_cnt, d_inv, d_out, d_residual};
     NX_TRY(launch_mfv(c, mp));
     return remember_routes();
   }

@@ -209,6 +209,17 @@ int launch_quantize(nx_ctx *c, int fmt, const float *d_src, size_t n, void *d_ds
 int launch_repack(nx_ctx *c, int fmt, const void *d_src, const RolePlane &pl, uint8_t *qs,
                   uint8_t *meta);
 
+// Rows of 256 activations to split into operand records (nx_split_dev.hpp).
+// The one-workgroup routing kernels take a job along on workgroups of their
+// own, where it costs no launch; `done` then.
+struct SplitJob {
+  const float *x;  // [n][256], 16-byte aligned
+  size_t n;
+  uint8_t *rec;    // [n] records
+  int fmt;
+  bool done;
+};
+
 int launch_route(nx_ctx *c, const float *d_logits, int T, int E, int k, int score_mode,
                  int32_t *d_expert, float *d_weight, int32_t *d_count);
 // d_tiles (optional): [0] = tile count, then (expert, first pair) per tile
@@ -217,7 +228,8 @@ int launch_route(nx_ctx *c, const float *d_logits, int T, int E, int k, int scor
 int launch_permute(nx_ctx *c, const int32_t *d_expert, const int32_t *d_count, int T, int k,
                    int E, int tile_m, int32_t *d_ecount, int32_t *d_offsets, int32_t *d_ptok,
                    int32_t *d_pslot, int32_t *d_inv, int32_t *d_active, int32_t *d_tiles,
-                   int shared_T, int tile_m2 = 0, int32_t *d_tiles2 = nullptr);
+                   int shared_T, int tile_m2 = 0, int32_t *d_tiles2 = nullptr,
+                   SplitJob *split = nullptr);
 // router + permutation in one workgroup, for small batches; d_tiles
 // (optional) as for launch_permute, without shared-expert tiles
 bool route_permute_fusable(int T, int E, int k);
@@ -225,7 +237,7 @@ int launch_route_permute(nx_ctx *c, const float *d_logits, int T, int E, int k, 
                          int32_t *d_expert, float *d_weight, int32_t *d_count, int32_t *d_ecount,
                          int32_t *d_offsets, int32_t *d_ptok, int32_t *d_pslot, int32_t *d_inv,
                          int32_t *d_active, int tile_m, int32_t *d_tiles, int *d_counters,
-                         int n_counters);
+                         int n_counters, SplitJob *split = nullptr);
 // logits[t][e] = sum_c w[e][c] x[t][c]; exact: the reference's sequential
 // order with separately rounded products and sums
 int launch_router_logits(nx_ctx *c, const float *d_w, const float *d_x, int T, int E, int H,
@@ -330,26 +342,28 @@ struct GemmPlan {
 // to the output in the combine (d_out may equal d_residual)
 int moe_forward(nx_ctx *c, const nx_experts *ex, const float *d_x, const float *d_logits, int T,
                 int k, int score_mode, int path, float *d_out, const float *d_residual);
-// few-token grouped matvec on MFMA (Q4_K): gate/up over K slices, SwiGLU of
-// the summed slices, down over K slices, then the combine (summing the down
+// few-token grouped matvec on MFMA: gate/up over K slices, SwiGLU of the
+// summed slices, down over K slices, then the combine (summing the down
 // slices in order) into out (+ residual)
 struct MfvPlan {
   const nx_experts *ex;
   int T, k;
-  const float *x;             // [T][H], 16-byte aligned
+  const uint8_t *rec;         // x's records, at mfv_records (a SplitJob)
   const int32_t *perm_token;  // [pairs]
   const int32_t *offsets;     // [E+1]
   const int32_t *tiles;       // tile list of the permutation with tile_m = kMfvTileM
-  int max_tiles;              // grid bound for the tile list
   const float *rw;            // combine inputs
   const int32_t *rcnt;
   const int32_t *inv;
   float *out;
   const float *residual;
 };
+size_t mfv_bytes(const nx_experts *ex, int T, int k);  // its workspace, but the routes'
+int mfv_records(nx_ctx *c, const nx_experts *ex, int T, int k, uint8_t **rec);
+int launch_mfv_split(nx_ctx *c, const SplitJob &job);
 int launch_mfv(nx_ctx *c, const MfvPlan &p);
-// whether the split-activation path takes these experts: Q4_K, or Q4_0
-// with hidden and FFN widths that are multiples of 256
+// whether the split-activation path takes these experts: Q4_K or Q2_K, or Q4_0
+// or Q8_0 with hidden and FFN widths that are multiples of 256
 bool mfv_supports(const nx_experts *ex);
 int mfv_max_tiles(int T, int k, int E, bool shared);
 constexpr int kMfvTileM = 16;

@@ -86,38 +86,6 @@ struct MfdStage {
   alignas(16) float sx[16];  // unscale factors
 };
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
-}
-
-// (q - 8) sc for the 8 codes of a dword holding q ^ 8, times 2^-14 (2^10 in
-// the scales) or any 2^k that keeps |.| fp16: s1 = {sc 2^(24+k)}, s16 = s1 / 16,
-// off = {-8 sc 2^k}
-__device__ __forceinline__ f16x8 operand4(uint32_t cw, f16x2 s1, f16x2 s16, f16x2 off) {
-  cw ^= 0x88888888u;
-  const uint32_t c8 = cw >> 8;
-  const f16x2 a = __builtin_bit_cast(f16x2, cw & 0x000F000Fu) * s1 + off;
-  const f16x2 b = __builtin_bit_cast(f16x2, cw & 0x00F000F0u) * s16 + off;
-  const f16x2 c = __builtin_bit_cast(f16x2, c8 & 0x000F000Fu) * s1 + off;
-  const f16x2 d = __builtin_bit_cast(f16x2, c8 & 0x00F000F0u) * s16 + off;
-  // a: elements 0, 2; c: 1, 3; b: 4, 6; d: 5, 7 (nibble 2 i of the dword is
-  // element i, nibble 2 i + 1 element 4 + i)
-  return f16x8{a[0], a[1], c[0], c[1], b[0], b[1], d[0], d[1]};
-}
-
-// q 2^-9 for the 8 signed bytes of two code dwords, in element order
-__device__ __forceinline__ f16x8 operand8(uint32_t lo, uint32_t hi) {
-  lo ^= 0x80808080u;
-  hi ^= 0x80808080u;
-  const f16x2 s = {32768.0f16, 32768.0f16}, off = {-0.25f16, -0.25f16};
-  const f16x2 a = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(lo, lo, 0x0C010C00u)) * s + off;
-  const f16x2 b = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(lo, lo, 0x0C030C02u)) * s + off;
-  const f16x2 c = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(hi, hi, 0x0C010C00u)) * s + off;
-  const f16x2 d = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(hi, hi, 0x0C030C02u)) * s + off;
-  return f16x8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
-}
-
 template <int FMT, int R, int KW>
 __global__ __launch_bounds__(64 * MD_WAVES, 2) void k_mfd(const MfdArgs a) {
   constexpr bool Q4K = FMT == NX_FMT_Q4_K, Q80 = FMT == NX_FMT_Q8_0;
@@ -179,61 +147,19 @@ __global__ __launch_bounds__(64 * MD_WAVES, 2) void k_mfd(const MfdArgs a) {
       for (int q = 0; q < 4; ++q)
         xr[p][q] = *reinterpret_cast<const f32x4 *>(xrow[p] + (size_t)c * MD_K + 64 * q);
   };
-  // elements 64 q + 4 l16 .. + 3 are half l16 % 2 of dword (l16 / 2) % 4 of
-  // sub-block (block) 2 q + l16 / 8
   auto stage_x = [&]() {
     Stage &st = sh.st[kg][rw];
-    const int kd = (l16 >> 1) & 3, s0 = l16 >> 3;
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       const int tok = 4 * p + g;
-      float mx = 0.f;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        // (fmaxf would first quiet each operand: two more instructions per pair)
-        asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(mx) : "v"(xr[p][q].x), "v"(xr[p][q].y));
-        asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(mx) : "v"(xr[p][q].z), "v"(xr[p][q].w));
-      }
-      mx = fmaxf(mx, dpp_f<0x128>(mx));  // row_ror 8, 4, 2, 1: the token's 16 lanes
-      mx = fmaxf(mx, dpp_f<0x124>(mx));
-      mx = fmaxf(mx, dpp_f<0x122>(mx));
-      mx = fmaxf(mx, dpp_f<0x121>(mx));
-      // max|x| < 2^E; an infinity or NaN ends as NaN through x' - hi or hi
-      int E = mx < INFINITY ? __builtin_amdgcn_frexp_expf(mx) : 0;
-      E = max(E, -100);
-      const float up = __builtin_amdgcn_ldexpf(1.0f, 14 - E);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        f16x2 h[2], l[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          // operand order of a 4-bit dword's half: elements 0, 2, 1, 3
-          const int e0 = Q80 ? 2 * i : i, e1 = Q80 ? 2 * i + 1 : i + 2;
-          h[i] = f16x2{(_Float16)(xr[p][q][e0] * up), (_Float16)(xr[p][q][e1] * up)};
-          asm("" : "+v"(h[i]));  // converted once: l reads the packed halves
-          l[i] = f16x2{(_Float16)fmaf(xr[p][q][e0], up, -(float)h[i][0]),
-                       (_Float16)fmaf(xr[p][q][e1], up, -(float)h[i][1])};
-        }
-        const int s = 2 * q + s0;
-        const int u = Q4K ? 4 * (s >> 2) + kd : s, gq = Q4K ? s & 3 : kd;
-        uint8_t *o = st.a + u * Stage::SU + gq * Stage::SG + 16 * tok + 8 * (l16 & 1);
-        *reinterpret_cast<f16x4 *>(o) = f16x4{h[0][0], h[0][1], h[1][0], h[1][1]};
-        *reinterpret_cast<f16x4 *>(o + Stage::SH) = f16x4{l[0][0], l[0][1], l[1][0], l[1][1]};
-        if constexpr (Q4K) {
-          // the sub-block's 8 lanes: quad pairs, quads, then the half row
-          float X = fmaf(xr[p][q].y, up, xr[p][q].x * up);
-          X = fmaf(xr[p][q].w, up, fmaf(xr[p][q].z, up, X));
-          X += dpp_f<0xB1>(X);
-          X += dpp_f<0x4E>(X);
-          X += dpp_f<0x141>(X);
-          const float xq = X * 0.015625f;  // |X| <= 32 x 2^14
-          const _Float16 xh = (_Float16)xq;
-          const f16x2 hl = {xh, (_Float16)(xq - (float)xh)};
-          // (its lanes hold the same sum and write the same word)
-          (&st.xm[tok + 16 * (s & 3)].x)[s >> 2] = __builtin_bit_cast(uint32_t, hl);
-        }
-      }
-      st.sx[tok] = __builtin_amdgcn_ldexpf(1.0f, E - 14);
+      st.sx[tok] = split16<FMT>(
+          xr[p], l16,
+          [&](int u, int gq, int half, f16x4 hi, f16x4 lo) {
+            uint8_t *o = st.a + u * Stage::SU + gq * Stage::SG + 16 * tok + 8 * half;
+            *reinterpret_cast<f16x4 *>(o) = hi;
+            *reinterpret_cast<f16x4 *>(o + Stage::SH) = lo;
+          },
+          [&](int gq, int i, f16x2 hl) { (&st.xm[tok + 16 * gq].x)[i] = __builtin_bit_cast(uint32_t, hl); });
     }
   };
   // between staging and use: the waves of a group share its stage
@@ -459,7 +385,7 @@ void (*mfd_pick(MfdShape s))(MfdArgs) {
 
 // From five tokens: the GEMV's time grows with every two tokens, and at five it
 // is behind at every size measured (us, GEMV / MFMA: 512 x 512 Q4_K 14.2 / 5.7,
-// 1024 x 2048 Q4_0 8.2 / 5.5, 4096 x 14336 Q4_K 45 / 26, 32000 x 4096 Q8_0 70 / 40);
+// 1024 x 2048 Q4_0 16.7 / 5.5, 4096 x 14336 Q4_K 45 / 26, 32000 x 4096 Q8_0 70 / 40);
 // up to four tokens a call gives each token the bits of a call of its own.
 bool mfd_takes(int fmt, const RolePlane &pl, const float *x, int T) {
   if (fmt != NX_FMT_Q4_K && fmt != NX_FMT_Q4_0 && fmt != NX_FMT_Q8_0) return false;

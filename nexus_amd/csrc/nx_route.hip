@@ -24,6 +24,7 @@
 #include "nx_device.hpp"
 #include "nx_internal.hpp"
 #include "nx_route_dev.hpp"
+#include "nx_split_dev.hpp"
 
 namespace nx {
 
@@ -83,7 +84,7 @@ __global__ __launch_bounds__(PERM_THREADS) void k_permute(
     int W, int tile_m, int32_t *__restrict__ ecount, int32_t *__restrict__ offsets,
     int32_t *__restrict__ ptok, int32_t *__restrict__ pslot, int32_t *__restrict__ inv,
     int32_t *__restrict__ active, int32_t *__restrict__ tiles, int shared_T, int tile_m2,
-    int32_t *__restrict__ tiles2) {
+    int32_t *__restrict__ tiles2, const SplitJob split) {
   __shared__ int cnt[PERM_THREADS];
   __shared__ int base[PERM_THREADS];
   __shared__ int run[PERM_THREADS];
@@ -91,6 +92,10 @@ __global__ __launch_bounds__(PERM_THREADS) void k_permute(
   __shared__ uint32_t pref[PERM_WORDS];
   __shared__ int wave_tot[PERM_THREADS / 64];
   __shared__ int total;
+  if (blockIdx.x > 0) {  // the split job's workgroups
+    split_rows(split, (size_t)(blockIdx.x - 1) * (PERM_THREADS / 16) + (threadIdx.x >> 4));
+    return;
+  }
   const int tid = threadIdx.x;
   for (int e = tid; e < E; e += PERM_THREADS) cnt[e] = 0;
   __syncthreads();
@@ -451,13 +456,18 @@ __global__ __launch_bounds__(RP_THREADS) void k_route_permute(
     int32_t *__restrict__ rexp, float *__restrict__ rw, int32_t *__restrict__ rcnt,
     int32_t *__restrict__ ecount, int32_t *__restrict__ offsets, int32_t *__restrict__ ptok,
     int32_t *__restrict__ pslot, int32_t *__restrict__ inv, int32_t *__restrict__ active,
-    int tile_m, int32_t *__restrict__ tiles, int *__restrict__ counters, int n_counters) {
+    int tile_m, int32_t *__restrict__ tiles, int *__restrict__ counters, int n_counters,
+    const SplitJob split) {
   __shared__ int s_exp[RP_MAX_PAIRS];
   __shared__ int s_cnt[RP_MAX_PAIRS];
   __shared__ int s_base[256];
   __shared__ uint32_t s_bits[256 * RP_WORDS];
   __shared__ int wave_tot[RP_THREADS / 64];
   __shared__ int total;
+  if (blockIdx.x > 0) {  // the split job's workgroups
+    split_rows(split, (size_t)(blockIdx.x - 1) * (RP_THREADS / 16) + (threadIdx.x >> 4));
+    return;
+  }
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int i = tid; i < n_counters; i += RP_THREADS) counters[i] = 0;
   for (int i = tid; i < E * RP_WORDS; i += RP_THREADS) s_bits[i] = 0;
@@ -936,10 +946,15 @@ int launch_route(nx_ctx *c, const float *d_logits, int T, int E, int k, int scor
 #undef NX_ROUTE
 }
 
+// workgroups of `threads` that a split job needs (16 threads per row)
+static unsigned split_blocks(const SplitJob &job, int threads) {
+  return (unsigned)((job.n * 16 + threads - 1) / threads);
+}
+
 int launch_permute(nx_ctx *c, const int32_t *d_expert, const int32_t *d_count, int T, int k,
                    int E, int tile_m, int32_t *d_ecount, int32_t *d_offsets, int32_t *d_ptok,
                    int32_t *d_pslot, int32_t *d_inv, int32_t *d_active, int32_t *d_tiles,
-                   int shared_T, int tile_m2, int32_t *d_tiles2) {
+                   int shared_T, int tile_m2, int32_t *d_tiles2, SplitJob *split) {
   if (E > PERM_THREADS) return fail(NX_ERR_UNSUPPORTED, "permutation supports at most 1024 experts");
   int W = PERM_WORDS / (E > 0 ? E : 1);
   if (W > PERM_THREADS / 32) W = PERM_THREADS / 32;
@@ -972,11 +987,13 @@ int launch_permute(nx_ctx *c, const int32_t *d_expert, const int32_t *d_count, i
       });
     }
   }
+  const SplitJob job = split ? *split : SplitJob{};
+  if (split) split->done = true;
   return launch(c, "permute", [&] {
-    go(c, k_permute, dim3(1), dim3(PERM_THREADS), 0, d_expert, d_count, T, k, E, W,
+    go(c, k_permute, dim3(1 + split_blocks(job, PERM_THREADS)), dim3(PERM_THREADS), 0, d_expert, d_count, T, k, E, W,
                                                  tile_m > 0 ? tile_m : 1, d_ecount, d_offsets,
                                                  d_ptok, d_pslot, d_inv, d_active, d_tiles,
-                                                 shared_T, tile_m2 > 0 ? tile_m2 : 1, d_tiles2);
+                                                 shared_T, tile_m2 > 0 ? tile_m2 : 1, d_tiles2, job);
   });
 }
 
@@ -994,17 +1011,20 @@ int launch_route_permute(nx_ctx *c, const float *d_logits, int T, int E, int k, 
                          int32_t *d_expert, float *d_weight, int32_t *d_count, int32_t *d_ecount,
                          int32_t *d_offsets, int32_t *d_ptok, int32_t *d_pslot, int32_t *d_inv,
                          int32_t *d_active, int tile_m, int32_t *d_tiles, int *d_counters,
-                         int n_counters) {
+                         int n_counters, SplitJob *split) {
   if (!route_permute_fusable(T, E, k)) return fail(NX_ERR_UNSUPPORTED, "batch too large for the fused router");
   const int epl = (E + 63) / 64;
   const int nc = d_counters ? n_counters : 0;
   const int tm = tile_m > 0 ? tile_m : 1;
+  const SplitJob job = split ? *split : SplitJob{};
+  if (split) split->done = true;
 #define NX_RP(N)                                                                              \
   return launch(c, "route_permute", [&] {                                                     \
-    go(c, k_route_permute<N>, dim3(1), dim3(RP_THREADS), 0, d_logits, T, E, k, score_mode, d_expert, \
+    go(c, k_route_permute<N>, dim3(1 + split_blocks(job, RP_THREADS)), dim3(RP_THREADS), 0, d_logits, \
+                                                        T, E, k, score_mode, d_expert, \
                                                         d_weight, d_count, d_ecount, d_offsets,  \
                                                         d_ptok, d_pslot, d_inv, d_active, tm,    \
-                                                        d_tiles, d_counters, nc);                \
+                                                        d_tiles, d_counters, nc, job);           \
   })
   if (epl <= 1) NX_RP(1);
   if (epl <= 2) NX_RP(2);
