@@ -29,9 +29,12 @@
 //                    4 instructions per 32 columns instead of 32, so a chain
 //                    advances one dependent add per instruction slot (about
 //                    4.4 clocks: a chain's latency is ~H * 1.9 ns).
-//   k_logits_tile    exact, many chains (prefill).  A workgroup owns a tile
-//                    of tokens x experts, each lane a register block of
-//                    chains, with both operands staged through an LDS ring.
+//   k_logits_tile    exact, more chains.  A workgroup owns a tile of tokens x
+//                    experts, each lane a chain, with both operands staged
+//                    through an LDS ring.
+//   k_logits_outer   exact, many chains (prefill).  Tiles of tokens x experts
+//                    whose products come from the matrix cores, one column at
+//                    a time, and are added in column order.
 //   k_logits_dot     fast, few tokens.  A workgroup per (expert, block of
 //                    tokens) strides over the row in 16-byte loads and reduces
 //                    with DPP and LDS.
@@ -464,21 +467,19 @@ __global__ __launch_bounds__(256) void k_block_prologue(const float *__restrict_
 
 constexpr int TL_NS = 3;  // ring stages of the tiled kernel
 
-// Tile of (16 RB tokens) x (16 RB experts) per 256-thread workgroup: lane l
-// holds the RB x RB chains of tokens t0 + RB (l / 16) + i and experts
-// e0 + RB (l % 16) + j.  Columns are staged KC = 128 / RB at a time (512
-// 16-byte units per operand and stage) in an LDS ring filled by DMA; unit u
-// of row r sits at r * (KC / 4) + (u ^ (r & 7)), so the rows a wave reads at
+// Tile of 16 tokens x 16 experts per 256-thread workgroup: lane l holds the
+// chain of token t0 + l / 16 and expert e0 + l % 16.  Columns are staged 128 at
+// a time (512 16-byte units per operand and stage) in an LDS ring filled by
+// DMA; unit u of row r sits at 32 r + (u ^ (r & 7)), so the rows a wave reads at
 // one column spread over the banks.  Each chain is summed in column order
 // with separately rounded products and sums (exact mode).
 // Requires H % 4 == 0 and 16-byte aligned rows.
-template <int RB>
 __global__ __launch_bounds__(256) void k_logits_tile(const float *__restrict__ W,
                                                      const float *__restrict__ X, int T, int E,
                                                      int H, float *__restrict__ out) {
 #pragma clang fp contract(off)
-  constexpr int ROWS = 16 * RB;   // rows per operand tile
-  constexpr int KC = 128 / RB;    // columns per stage
+  constexpr int ROWS = 16;        // rows per operand tile
+  constexpr int KC = 128;         // columns per stage
   constexpr int U = KC / 4;       // 16-byte units per row
   constexpr int UNITS = ROWS * U; // = 512
   // 1 KB DMAs per operand and stage: UNITS / 64 = 8, two per wave
@@ -533,36 +534,17 @@ __global__ __launch_bounds__(256) void k_logits_tile(const float *__restrict__ W
   };
 
   const int tg = tid >> 4, eg = tid & 15;
-  float s[RB][RB];
-#pragma unroll
-  for (int i = 0; i < RB; ++i)
-#pragma unroll
-    for (int j = 0; j < RB; ++j) s[i][j] = 0.f;
+  float s = 0.f;
   auto compute = [&](auto st) {
     const float *wb = wbuf(st), *xb = xbuf(st);
 #pragma unroll
     for (int k4 = 0; k4 < U; ++k4) {
-      float4 xv[RB], wv[RB];
-#pragma unroll
-      for (int i = 0; i < RB; ++i) {
-        const int r = RB * tg + i;
-        xv[i] = *reinterpret_cast<const float4 *>(xb + 4 * (r * U + (k4 ^ (r & 7))));
-      }
-#pragma unroll
-      for (int j = 0; j < RB; ++j) {
-        const int r = RB * eg + j;
-        wv[j] = *reinterpret_cast<const float4 *>(wb + 4 * (r * U + (k4 ^ (r & 7))));
-      }
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-        for (int i = 0; i < RB; ++i)
-#pragma unroll
-          for (int j = 0; j < RB; ++j) {
-            const float xk = kk == 0 ? xv[i].x : kk == 1 ? xv[i].y : kk == 2 ? xv[i].z : xv[i].w;
-            const float wk = kk == 0 ? wv[j].x : kk == 1 ? wv[j].y : kk == 2 ? wv[j].z : wv[j].w;
-            s[i][j] = s[i][j] + wk * xk;
-          }
+      const float4 xv = *reinterpret_cast<const float4 *>(xb + 4 * (tg * U + (k4 ^ (tg & 7))));
+      const float4 wv = *reinterpret_cast<const float4 *>(wb + 4 * (eg * U + (k4 ^ (eg & 7))));
+      s = s + wv.x * xv.x;
+      s = s + wv.y * xv.y;
+      s = s + wv.z * xv.z;
+      s = s + wv.w * xv.w;
     }
   };
   // stage c: wait for its DMA (stage c+1 may stay in flight), barrier (all
@@ -586,15 +568,8 @@ __global__ __launch_bounds__(256) void k_logits_tile(const float *__restrict__ W
     step(IC<2>{}, c + 2);
   }
   wait_vm<0>();  // the DMA of stages past the end has drained
-#pragma unroll
-  for (int i = 0; i < RB; ++i) {
-    const int t = t0 + RB * tg + i;
-#pragma unroll
-    for (int j = 0; j < RB; ++j) {
-      const int e = e0 + RB * eg + j;
-      if (t < T && e < E) out[(size_t)t * E + e] = s[i][j];
-    }
-  }
+  const int t = t0 + tg, e = e0 + eg;
+  if (t < T && e < E) out[(size_t)t * E + e] = s;
 }
 
 // fast mode, few tokens: workgroup (expert, token block of BT)
@@ -813,13 +788,94 @@ __global__ __launch_bounds__(256) void k_logits_mfma(const float *__restrict__ W
     }
 }
 
-void launch_tile(nx_ctx *c, int rb, const float *W, const float *X, int T, int E, int H,
-                 float *out) {
-  const int rows = 16 * rb;
-  const dim3 grid((E + rows - 1) / rows, (T + rows - 1) / rows);
-  if (rb == 4) go(c, k_logits_tile<4>, dim3(grid), dim3(256), 0, W, X, T, E, H, out);
-  else if (rb == 2) go(c, k_logits_tile<2>, dim3(grid), dim3(256), 0, W, X, T, E, H, out);
-  else go(c, k_logits_tile<1>, dim3(grid), dim3(256), 0, W, X, T, E, H, out);
+// Tile of 32 tokens x 32 experts per 256-thread workgroup, 16 x 16 per wave:
+// lane l holds the chains of tokens 4 (l / 16) + r (r = 0..3) and expert l % 16
+// of the wave's tile.  v_mfma_f32_16x16x1_4b_f32 on a zero accumulator gives the
+// rounded products of four consecutive columns (one per block) of all 256
+// chains, so the vector ALU only adds them, in column order: the separately
+// rounded products and sums of exact mode.  Columns are staged 64 at a time
+// in two LDS buffers filled by DMA; the 16-byte unit u of row r sits at
+// 256 r + 16 (u ^ (r % 16)), so a wave's reads (16 rows x 4 columns) take every
+// bank once.
+// Bound by the adds: 16 per 4 columns and wave, 191 us of issue at 4096 tokens
+// x 256 experts x 7168 columns on one MI355X.  With products and sums both on
+// the vector ALU (4 x 4 chains per lane, one wave per SIMD) that took 843 us,
+// now 322 us.
+// Requires H % 4 == 0 and 16-byte aligned rows.
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+__global__ __launch_bounds__(256, 4) void k_logits_outer(const float *__restrict__ W,
+                                                         const float *__restrict__ X, int T, int E,
+                                                         int H, float *__restrict__ out) {
+#pragma clang fp contract(off)
+  constexpr int ROWS = 32, KC = 64;
+  __shared__ __attribute__((aligned(16))) float w0[ROWS * KC], x0[ROWS * KC];
+  __shared__ __attribute__((aligned(16))) float w1[ROWS * KC], x1[ROWS * KC];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int e0 = blockIdx.x * ROWS, t0 = blockIdx.y * ROWS;
+  // the workgroup's own rows: rows past the matrix lie past the range
+  const auto rw = make_rsrc(W + (size_t)e0 * H, (uint32_t)min(ROWS, E - e0) * (uint32_t)H * 4u);
+  const auto rx = make_rsrc(X + (size_t)t0 * H, (uint32_t)min(ROWS, T - t0) * (uint32_t)H * 4u);
+  // DMA d (0..7) of an operand fills rows 4 d .. 4 d + 3; wave w issues d = 2 w
+  // and 2 w + 1 of both
+  uint32_t doff[2];
+  int dcol[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = 4 * (2 * wave + i) + (lane >> 4), u = (lane & 15) ^ (r & 15);
+    doff[i] = (uint32_t)r * (uint32_t)H * 4u + 16u * (uint32_t)u;
+    dcol[i] = 4 * u;
+  }
+  auto issue = [&](float *wb, float *xb, int c) {
+    const int k0 = c * KC;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t off = k0 + dcol[i] < H ? doff[i] + 4u * (uint32_t)k0 : OOB;
+      const int dst = (2 * wave + i) * 256;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_void *)(wb + dst), 16, off, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void *)(xb + dst), 16, off, 0, 0, 0);
+    }
+  };
+  const int l16 = lane & 15, b = lane >> 4;
+  const int rt = 16 * (wave >> 1), re = 16 * (wave & 1);
+  int col[16];  // float index of column 4 k4 + b in row l16
+#pragma unroll
+  for (int k4 = 0; k4 < 16; ++k4) col[k4] = l16 * KC + 4 * (k4 ^ l16) + b;
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](const float *wb, const float *xb) {
+    const f32x16_t zero = {};
+    f32x16_t p[2];
+    p[0] = __builtin_amdgcn_mfma_f32_16x16x1f32(xb[rt * KC + col[0]], wb[re * KC + col[0]], zero, 0, 0, 0);
+#pragma unroll
+    for (int k4 = 0; k4 < 16; ++k4) {
+      if (k4 < 15)
+        p[(k4 + 1) & 1] = __builtin_amdgcn_mfma_f32_16x16x1f32(xb[rt * KC + col[k4 + 1]], wb[re * KC + col[k4 + 1]],
+                                                               zero, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i & 3] = s[i & 3] + p[k4 & 1][i];
+    }
+  };
+  // stage c: its DMA has landed for all waves, and all are done with stage
+  // c - 1's buffer, which then takes stage c + 1
+  const int nst = (H + KC - 1) / KC;
+  issue(w0, x0, 0);
+  for (int c = 0; c < nst; c += 2) {
+    wait_vm<0>();
+    lds_barrier();
+    issue(w1, x1, c + 1);
+    compute(w0, x0);
+    if (c + 1 >= nst) break;
+    wait_vm<0>();
+    lds_barrier();
+    issue(w0, x0, c + 2);
+    compute(w1, x1);
+  }
+  wait_vm<0>();  // the DMA of a stage past the end has drained
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int t = t0 + rt + 4 * b + r, e = e0 + re + l16;
+    if (t < T && e < E) out[(size_t)t * E + e] = s[r];
+  }
 }
 
 }  // namespace
@@ -908,10 +964,18 @@ int launch_router_logits(nx_ctx *c, const float *d_w, const float *d_x, int T, i
       else go(c, k_logits_mfma<2, 2, 4>, grid, dim3(256), 0, d_w, d_x, T, E, H, d_out);
     });
   }
-  // chains per lane: as many as keep at least 1024 waves in the grid
-  const int rb = chains >= 1024L * 64 * 16 ? 4 : (chains >= 1024L * 64 * 4 ? 2 : 1);
+  // a wave of k_logits_outer holds 256 chains and one of k_logits_tile 64: the
+  // former from the count that gives every SIMD a wave (us, against tiles of 2
+  // x 2 or 4 x 4 chains per lane: 1024 x 256 x 7168 214 -> 122, 2048 x 128 x 2048
+  // 59 -> 40, 32768 x 8 x 4096, half of each tile empty, 326 -> 169)
+  if (chains >= 1024L * 256) {
+    const dim3 grid((E + 31) / 32, (T + 31) / 32);
+    return launch(c, "router_logits_outer",
+                  [&] { go(c, k_logits_outer, grid, dim3(256), 0, d_w, d_x, T, E, H, d_out); });
+  }
+  const dim3 grid((E + 15) / 16, (T + 15) / 16);
   return launch(c, "router_logits_tile",
-                [&] { launch_tile(c, rb, d_w, d_x, T, E, H, d_out); });
+                [&] { go(c, k_logits_tile, grid, dim3(256), 0, d_w, d_x, T, E, H, d_out); });
 }
 
 int launch_block_prologue(nx_ctx *c, const float *d_x, const float *d_nw, float eps,
