@@ -87,11 +87,11 @@ extern "C" {
 #define NX_SCORE_SIGMOID 1 /* extension: sigmoid scores renormalised over the top-k */
 
 /* expert-product paths */
-#define NX_PATH_AUTO 0      /* by tokens per expert: GEMV, then (Q4_K and Q2_K with no shared
-                               expert or one as wide as the routed experts; Q4_0 and Q8_0 in
-                               whole 256-weight chunks with no shared expert) the
-                               split-activation MFMA path, then (not Q2_K) the grouped GEMM
-                               on bf16 operands */
+#define NX_PATH_AUTO 0      /* by tokens per expert and the layer's size: GEMV, then (Q4_K and
+                               Q2_K, and Q4_0 and Q8_0 in whole 256-weight chunks; with no
+                               shared expert or one as wide as the routed experts, Q4_0 and
+                               Q8_0 there only in large layers) the split-activation MFMA
+                               path, then (not Q2_K) the grouped GEMM on bf16 operands */
 #define NX_PATH_GEMV 1      /* dequant-in-register GEMV, fp32 accumulate */
 #define NX_PATH_MFMA_F16 2  /* grouped GEMM on fp16 MFMA, fp32 accumulate; activations and
                                SwiGLU outputs must stay within fp16's range (|v| < 65504) */
@@ -226,7 +226,9 @@ int nx_matrix_destroy(nx_matrix *m);
 /* y[t * rows + r] = sum_c W[r][c] x[t * cols + c] for T = num_tokens, fp32
  * in and out: InferenceEngine::matvec (src/engine/mod.rs:775-801) on each
  * token row, with the dot product in parallel order (fp32 accumulate) over
- * weights dequantized in registers.  x_len != T*cols gives NX_ERR_SHAPE
+ * the quantized codes.  Five and more tokens of Q4_K, Q4_0 or Q8_0 rows of
+ * whole 256-weight chunks run on the matrix cores, within the same error, so a
+ * token's last bits can differ between the two.  x_len != T*cols gives NX_ERR_SHAPE
  * "Matvec input shape mismatch: got <x_len>, expected <T*cols>". */
 int nx_matvec(nx_ctx *ctx, const nx_matrix *m, const float *x, size_t x_len, int num_tokens,
               float *y);
