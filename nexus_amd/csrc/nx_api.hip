@@ -1083,10 +1083,10 @@ int nx::moe_forward(nx_ctx *c, const nx_experts *ex, const float *d_x, const flo
     uint8_t *d_rec;
     NX_TRY(mfv_records(c, ex, T, k, &d_rec));
     SplitJob split{d_x, (size_t)T * H / 256, d_rec, ex->fmt, false};
-    // (the fused router lists no shared-expert tiles)
-    if (!shared && route_permute_fusable(T, E, k)) {
+    if (route_permute_fusable(T, E, k)) {
       NX_TRY(launch_route_permute(c, d_logits, T, E, k, score_mode, d_exp, d_w, d_cnt, d_ec, d_off,
-                                  d_pt, d_ps, d_inv, d_act, kMfvTileM, d_tiles, nullptr, 0, &split));
+                                  d_pt, d_ps, d_inv, d_act, kMfvTileM, d_tiles, nullptr, 0,
+                                  shared ? T : 0, &split));
     } else {
       NX_TRY(launch_route(c, d_logits, T, E, k, score_mode, d_exp, d_w, d_cnt));
       NX_TRY(launch_permute(c, d_exp, d_cnt, T, k, E, kMfvTileM, d_ec, d_off, d_pt, d_ps, d_inv,
