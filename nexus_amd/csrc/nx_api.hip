@@ -956,89 +956,8 @@ int nx::moe_forward(nx_ctx *c, const nx_experts *ex, const float *d_x, const flo
     return fail(NX_ERR_UNSUPPORTED,
                 "Q2_K experts run on the GEMV and the split-activation MFMA path only");
   }
-  // AUTO takes bf16 operands on the grouped GEMM: fp16's range ends at
-  // 65504, which SwiGLU activations of real models can pass; bf16 keeps
-  // float32's range, runs as fast here, and stays within the MFMA bar.
-  if (use == NX_PATH_AUTO) {
-    // Tokens per active expert, with the active count expected under
-    // uniform routing, E (1 - (1 - k/E)^T).
-    const double kk = std::min(1.0, (double)k / E);
-    const double act = std::max(1.0, E * (1.0 - std::pow(1.0 - kk, (double)T)));
-    const double tpe = (double)T * k / act;
-    // The split path streams the active experts' weights at 4.3 TB/s behind
-    // about 35 us of launches, so it wins over wider ranges where an expert is
-    // large: `large` from 7 M weights a matrix (measured at 4096 x 1792 and up).
-    // In the fixed scratch array of nx_moe_forward_noalloc a batch that its
-    // workspace would not fit keeps the narrower ranges, whose other paths
-    // need less.
-    const bool fits = !c->scratch_mode ||
-                      mfv_bytes(ex, T, k) + (size_t)T * k * 64 + (size_t)E * 64 + (1u << 20) <= kScratchBytes;
-    const double weights = (double)H * ex->F;
-    const bool large = fits && weights >= 7e6;
-    const bool q8 = ex->fmt == NX_FMT_Q8_0;
-    const bool split_fmt = ex->fmt == NX_FMT_Q4_K || ((ex->fmt == NX_FMT_Q4_0 || q8) && mfv_supports(ex));
-    if (ex->fmt == NX_FMT_Q2_K) {
-      // The GEMV or the split-activation path (Q2_K has no grouped GEMM).
-      // Measured (ms, GEMV / split): Mixtral 2 tokens 0.101 / 0.122, 4:
-      // 0.173 / 0.188, 8: 0.243 / 0.193, 32: 0.939 / 0.238, 128: 2.82 /
-      // 0.534; Qwen3 4 tokens 0.048 / 0.048, 8: 0.093 / 0.065, 512: 1.84 /
-      // 0.265; DeepSeek with its shared expert 2 tokens 0.119 / 0.137, 4:
-      // 0.307 / 0.218, 64: 44.1 / 1.52.
-      if (shared)
-        use = (ex->Fs == ex->F && T >= 4) ? NX_PATH_MFMA_SPLIT : NX_PATH_GEMV;
-      else
-        use = (tpe >= 1.8 || ((long)T * k >= 64 && tpe >= 1.2)) ? NX_PATH_MFMA_SPLIT
-                                                                 : NX_PATH_GEMV;
-    } else if (split_fmt && shared && ex->Fs == ex->F && (large || ex->fmt == NX_FMT_Q4_K)) {
-      // A shared expert sees every token: the GEMV walks it a token pair at
-      // a time, the split-activation path 16 tokens at a time.  Measured
-      // (DeepSeek shapes, us, GEMV / split / grouped GEMM): Q4_K 2 tokens 105
-      // / 128 / 233, 4: 265 / 196 / 282, 27: 9257 / 836 / 1251, 128: - / 1546 /
-      // 1989, 256 (8 per routed expert): - / 1836 / 2090, 400 (12.5): - / 2105
-      // / 2123; Q4_0 4: 232 / 198 / 281, 27: - / 950 / 1226, 128: - / 1665 /
-      // 1960; Q8_0 8: 840 / 542 / 643, 27: - / 1357
-      // / 1524, 300 (9.4): - / 2924 / 2730.
-      if (tpe >= (large && !q8 ? 12.0 : 8.0))
-        use = NX_PATH_MFMA_BF16;
-      else
-        use = T >= (q8 ? 6 : 4) ? NX_PATH_MFMA_SPLIT : NX_PATH_GEMV;
-    } else if (split_fmt && !shared) {
-      // The GEMV re-reads an expert's weights per pair of its tokens, the
-      // split-activation path reads them once per 16 tokens, and the grouped
-      // GEMM once, at bf16 operands.  Measured (us, GEMV / split / grouped
-      // GEMM) by tokens per expert: Mixtral Q4_0 1.1: 80 / 96 / 176, 1.5: 154 /
-      // 130 / 240, 2.0: 249 / 155 / 244; Q4_K 1.3: 128 / 107 / 201, 2.2: 454 /
-      // 156 / 254, 8: 906 / 215 / 301, 12: - / 241 / 304, 16: - / 320 / 305;
-      // Q8_0 2.0: 320 / 239 / 295, 8: - / 338 / 363, 16: - / 540 / 365; Qwen3
-      // Q4_K 1.1: 45 / 50 / 68, 1.3: 107 / 64 / 93, 8: - / 132 / 151, 12.5: -
-      // / 137 / 153, 16: - / 155 / 156.  Smaller layers (GEMV / split): 8
-      // experts of 4096 x 1792 Q4_K 1.3: 38 / 37, 1.6: 57 / 43, Q8_0 1.6: 48 /
-      // 54, 2.2: 59 / 54; 1024 x 2048 Q4_K 1.3: 31 / 35, 1.6: 42 / 35; 512 x
-      // 1024 Q4_K 1.6: 25 / 34, 2.2: 35 / 36, 3.1: 46 / 37; 64 experts of 1024
-      // x 768, top 8, 1.1: 35 / 35, 1.3: 53 / 36.
-      const long pairs = (long)T * k;
-      if (tpe >= (large && !q8 ? 13.0 : 12.0))
-        use = NX_PATH_MFMA_BF16;
-      else if (tpe >= 3.0 || (pairs >= 64 && tpe >= 1.2) || (fits && pairs >= 40 && tpe >= 1.25) ||
-               (large && tpe >= (q8 ? 2.0 : 1.28)) || (fits && !q8 && weights >= 2e6 && tpe >= 1.6))
-        use = NX_PATH_MFMA_SPLIT;
-      else
-        use = NX_PATH_GEMV;
-    } else if (ex->fmt == NX_FMT_F32) {
-      // f32 weights keep their precision on the GEMV; the bf16 grouped GEMM
-      // only once experts see 32 tokens on average
-      const long active_max = std::min<long>(E, (long)T * k);
-      use = ((long)T * k >= 32 * active_max) ? NX_PATH_MFMA_BF16 : NX_PATH_GEMV;
-    } else {
-      // The grouped GEMM from ~3 tokens per routed expert (Mixtral Q8_0 and
-      // Q4_0 at 8 and 16 tokens, Qwen3 Q8_0 at 32), or from 6 tokens when a
-      // shared expert sees them all: the GEMV passes over the shared expert
-      // per pair of tokens and over the routed experts per token group
-      // (DeepSeek shapes with a shared expert: GEMV 0.29 / 0.81 / 10.5 ms
-      // at 4 / 8 / 32 tokens, grouped GEMM 0.36 / 0.61 / 1.44 ms).
-      use = (tpe >= 3.0 || (shared && T >= 6)) ? NX_PATH_MFMA_BF16 : NX_PATH_GEMV;
-    }
-  }
+  if (use == NX_PATH_AUTO)
+    use = auto_path(shape_of(ex), T, k, c->scratch_mode ? kScratchBytes : SIZE_MAX);
 
   if (use == NX_PATH_GEMV) {
     NX_TRY(ws(c, WS_YPAIR, pairs_total * H, &d_ypair));
@@ -1067,10 +986,10 @@ int nx::moe_forward(nx_ctx *c, const nx_experts *ex, const float *d_x, const flo
   }
 
   if (use == NX_PATH_MFMA_SPLIT) {
-    if (!mfv_supports(ex))
+    if (!mfv_supports(shape_of(ex)))
       return fail(NX_ERR_UNSUPPORTED,
-                  "the split-activation MFMA path takes Q4_K experts, or Q4_0 experts whose "
-                  "hidden and FFN widths are multiples of 256");
+                  "the split-activation MFMA path takes Q4_K and Q2_K experts, or Q4_0 and Q8_0 "
+                  "experts whose hidden and FFN widths are multiples of 256");
     if (shared && ex->Fs != ex->F)
       return fail(NX_ERR_UNSUPPORTED,
                   "the split-activation MFMA path takes a shared expert as wide as the routed ones");

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "../../include/nexus_hip.h"
+#include "nx_plan.hpp"
 
 namespace nx {
 
@@ -134,6 +135,8 @@ struct nx_experts {
 };
 
 namespace nx {
+
+inline MoeShape shape_of(const nx_experts *ex) { return {ex->fmt, ex->E, ex->H, ex->F, ex->Fs}; }
 
 // workspace slots
 enum WsSlot {
@@ -358,13 +361,9 @@ struct MfvPlan {
   float *out;
   const float *residual;
 };
-size_t mfv_bytes(const nx_experts *ex, int T, int k);  // its workspace, but the routes'
 int mfv_records(nx_ctx *c, const nx_experts *ex, int T, int k, uint8_t **rec);
 int launch_mfv_split(nx_ctx *c, const SplitJob &job);
 int launch_mfv(nx_ctx *c, const MfvPlan &p);
-// whether the split-activation path takes these experts: Q4_K or Q2_K, or Q4_0
-// or Q8_0 with hidden and FFN widths that are multiples of 256
-bool mfv_supports(const nx_experts *ex);
 int mfv_max_tiles(int T, int k, int E, bool shared);
 constexpr int kMfvTileM = 16;
 // grouped-GEMM M-tile height of a pass for a batch

@@ -56,7 +56,6 @@ namespace nx {
 namespace {
 
 constexpr int MV_M = 16;   // pairs per tile
-constexpr int MV_K = 256;  // K positions per chunk
 
 struct MfvArgs {
   const uint8_t *qs0, *qs1, *meta0, *meta1;  // role planes (gate, up) or (down, -)
@@ -91,7 +90,6 @@ struct MfvStep {
 };
 
 constexpr int MV_STEPS = 8;  // (row tile, matrix) steps per pass of the loop
-constexpr int MV_KW = 8;     // chunks per K slice, at most: one per wave
 constexpr int MV_D = 4;      // steps in flight (2, 3 or 6: within 3%)
 
 template <bool GATEUP, int FMT>
@@ -393,29 +391,12 @@ __global__ __launch_bounds__(256) void k_mfv_swiglu(const float *__restrict__ pa
   if (i < n) write_record<FMT>(rec + i * REC_BYTES, v, j);
 }
 
-// Chunks per K slice: as many slices of at most MV_KW chunks as the row needs,
-// of equal size (but for the last one's remainder)
-int mv_slice_chunks(int nchunk) {
-  const int n = (nchunk + MV_KW - 1) / MV_KW;
-  return (nchunk + n - 1) / n;
-}
-
-// Both passes' partial sums share one buffer: the down pass writes it after
-// the gate/up sums, and x's records behind them, are dead.
-struct MfvSizes {
-  size_t pairs;
-  int ks_g, ks_d, nks_g, nks_d;  // chunks per K slice, slices
-  size_t gate, part, recs;       // bytes: gate/up sums, the shared buffer, the gated rows' records
-};
-
-MfvSizes mfv_sizes(const nx_experts *ex, int T, int k);
-
 template <int FMT>
 int run_mfv(nx_ctx *c, const MfvPlan &p) {
   const nx_experts *ex = p.ex;
   const bool shared = ex->Fs > 0;
   const int H = ex->H, F = ex->F, cd = F / MV_K;
-  const MfvSizes z = mfv_sizes(ex, p.T, p.k);
+  const MfvSizes z = mfv_sizes(shape_of(ex), p.T, p.k);
   const size_t pairs = z.pairs;
   const int nks_g = z.nks_g, nks_d = z.nks_d;
   void *vp, *vr;
@@ -480,22 +461,6 @@ int run_mfv(nx_ctx *c, const MfvPlan &p) {
                         pairs * (size_t)H, p.residual);
 }
 
-MfvSizes mfv_sizes(const nx_experts *ex, int T, int k) {
-  // routed pairs, then one pair per token for the shared expert
-  const size_t pairs = (size_t)T * k + (ex->Fs > 0 ? (size_t)T : 0);
-  const int cg = ex->H / MV_K, cd = ex->F / MV_K;
-  MfvSizes z{};
-  z.pairs = pairs;
-  z.ks_g = mv_slice_chunks(cg);
-  z.ks_d = mv_slice_chunks(cd);
-  z.nks_g = (cg + z.ks_g - 1) / z.ks_g;
-  z.nks_d = (cd + z.ks_d - 1) / z.ks_d;
-  z.gate = (size_t)z.nks_g * pairs * 2 * ex->F * sizeof(float);
-  z.part = std::max(z.gate + (size_t)T * cg * REC_BYTES, (size_t)z.nks_d * pairs * ex->H * sizeof(float));
-  z.recs = pairs * cd * REC_BYTES;
-  return z;
-}
-
 }  // namespace
 
 int mfv_max_tiles(int T, int k, int E, bool shared) {
@@ -504,21 +469,8 @@ int mfv_max_tiles(int T, int k, int E, bool shared) {
                (shared ? (T + MV_M - 1) / MV_M : 0));
 }
 
-bool mfv_supports(const nx_experts *ex) {
-  // whole 256-weight chunks in both products: Q4_K and Q2_K always, Q4_0
-  // and Q8_0 when H and F are multiples of 256
-  if (ex->fmt == NX_FMT_Q4_K || ex->fmt == NX_FMT_Q2_K) return true;
-  return (ex->fmt == NX_FMT_Q4_0 || ex->fmt == NX_FMT_Q8_0) && ex->H % MV_K == 0 &&
-         ex->F % MV_K == 0;
-}
-
-size_t mfv_bytes(const nx_experts *ex, int T, int k) {
-  const MfvSizes z = mfv_sizes(ex, T, k);
-  return z.part + z.recs;
-}
-
 int mfv_records(nx_ctx *c, const nx_experts *ex, int T, int k, uint8_t **rec) {
-  const MfvSizes z = mfv_sizes(ex, T, k);
+  const MfvSizes z = mfv_sizes(shape_of(ex), T, k);
   void *p;
   NX_TRY(ws_get(c, WS_MFV_PART, z.part, &p));
   *rec = static_cast<uint8_t *>(p) + z.gate;
@@ -533,7 +485,7 @@ int launch_mfv_split(nx_ctx *c, const SplitJob &job) {
 
 int launch_mfv(nx_ctx *c, const MfvPlan &p) {
   const nx_experts *ex = p.ex;
-  if (!mfv_supports(ex))
+  if (!mfv_supports(shape_of(ex)))
     return fail(NX_ERR_UNSUPPORTED,
                 "the split-activation MFMA path takes Q4_K and Q2_K experts, or Q4_0 and Q8_0 "
                 "experts whose hidden and FFN widths are multiples of 256");

@@ -1,0 +1,157 @@
+// nx_plan.hpp — what a MoE call's sizes alone decide: the path AUTO takes and
+// the split-activation path's workspace.
+//
+// Plain C++ (no HIP): the CPU tests compile this header on its own.
+#pragma once
+
+#include <algorithm>
+#include <cmath>
+#include <cstddef>
+#include <cstdint>
+
+#include "../../include/nexus_hip.h"
+
+namespace nx {
+
+// an expert layer's format and widths (Fs: the shared expert's, or 0)
+struct MoeShape {
+  int fmt, E, H, F, Fs;
+};
+
+// ---- split-activation path (nx_mfv.hip)
+constexpr int MV_K = 256;        // K positions per chunk
+constexpr int MV_KW = 8;         // chunks per K slice, at most: one per wave
+constexpr int REC_BYTES = 1152;  // operand record of a row's chunk (nx_split_dev.hpp)
+
+// whether the path takes these experts: whole 256-weight chunks in both
+// products (Q4_K and Q2_K always)
+inline bool mfv_supports(const MoeShape &s) {
+  if (s.fmt == NX_FMT_Q4_K || s.fmt == NX_FMT_Q2_K) return true;
+  return (s.fmt == NX_FMT_Q4_0 || s.fmt == NX_FMT_Q8_0) && s.H % MV_K == 0 && s.F % MV_K == 0;
+}
+
+// Chunks per K slice: as many slices of at most MV_KW chunks as the row needs,
+// of equal size (but for the last one's remainder)
+inline int mv_slice_chunks(int nchunk) {
+  if (nchunk <= 0) return 1;  // (no such layer is supported)
+  const int n = (nchunk + MV_KW - 1) / MV_KW;
+  return (nchunk + n - 1) / n;
+}
+
+// Both passes' partial sums share one buffer: the down pass writes it after
+// the gate/up sums, and x's records behind them, are dead.
+struct MfvSizes {
+  size_t pairs;
+  int ks_g, ks_d, nks_g, nks_d;  // chunks per K slice, slices
+  size_t gate, part, recs;       // bytes: gate/up sums, the shared buffer, the gated rows' records
+};
+
+inline MfvSizes mfv_sizes(const MoeShape &s, int T, int k) {
+  // routed pairs, then one pair per token for the shared expert
+  const size_t pairs = (size_t)T * k + (s.Fs > 0 ? (size_t)T : 0);
+  const int cg = s.H / MV_K, cd = s.F / MV_K;
+  MfvSizes z{};
+  z.pairs = pairs;
+  z.ks_g = mv_slice_chunks(cg);
+  z.ks_d = mv_slice_chunks(cd);
+  z.nks_g = (cg + z.ks_g - 1) / z.ks_g;
+  z.nks_d = (cd + z.ks_d - 1) / z.ks_d;
+  z.gate = (size_t)z.nks_g * pairs * 2 * s.F * sizeof(float);
+  z.part = std::max(z.gate + (size_t)T * cg * REC_BYTES, (size_t)z.nks_d * pairs * s.H * sizeof(float));
+  z.recs = pairs * cd * REC_BYTES;
+  return z;
+}
+
+// its workspace, but the routes'
+inline size_t mfv_bytes(const MoeShape &s, int T, int k) {
+  const MfvSizes z = mfv_sizes(s, T, k);
+  return z.part + z.recs;
+}
+
+// ---- AUTO
+// The path of a call on T tokens, top k.  scratch: the bytes its workspace may
+// take (SIZE_MAX where it is allocated).
+//
+// AUTO takes bf16 operands on the grouped GEMM: fp16's range ends at 65504,
+// which SwiGLU activations of real models can pass; bf16 keeps float32's range,
+// runs as fast here, and stays within the MFMA bar.
+inline int auto_path(const MoeShape &s, int T, int k, size_t scratch) {
+  if (s.fmt == NX_FMT_F16 || s.fmt == NX_FMT_BF16) return NX_PATH_GEMV;
+  const bool shared = s.Fs > 0;
+  // Tokens per active expert, with the active count expected under
+  // uniform routing, E (1 - (1 - k/E)^T).
+  const double kk = std::min(1.0, (double)k / s.E);
+  const double act = std::max(1.0, s.E * (1.0 - std::pow(1.0 - kk, (double)T)));
+  const double tpe = (double)T * k / act;
+  // The split path streams the active experts' weights at 4.3 TB/s behind
+  // about 35 us of launches, so it wins over wider ranges where an expert is
+  // large: `large` from 7 M weights a matrix (measured at 4096 x 1792 and up).
+  // In the fixed scratch array of nx_moe_forward_noalloc a batch that its
+  // workspace would not fit keeps the narrower ranges, whose other paths
+  // need less.
+  const bool split_fmt = mfv_supports(s);
+  const bool fits = split_fmt && (scratch == SIZE_MAX || mfv_bytes(s, T, k) + (size_t)T * k * 64 +
+                                                                 (size_t)s.E * 64 + (1u << 20) <=
+                                                             scratch);
+  const double weights = (double)s.H * s.F;
+  const bool large = fits && weights >= 7e6;
+  const bool q8 = s.fmt == NX_FMT_Q8_0;
+  if (s.fmt == NX_FMT_Q2_K) {
+    // The GEMV or the split-activation path (Q2_K has no grouped GEMM).
+    // Measured (ms, GEMV / split): Mixtral 2 tokens 0.101 / 0.122, 4:
+    // 0.173 / 0.188, 8: 0.243 / 0.193, 32: 0.939 / 0.238, 128: 2.82 /
+    // 0.534; Qwen3 4 tokens 0.048 / 0.048, 8: 0.093 / 0.065, 512: 1.84 /
+    // 0.265; DeepSeek with its shared expert 2 tokens 0.119 / 0.137, 4:
+    // 0.307 / 0.218, 64: 44.1 / 1.52.
+    if (shared) return (s.Fs == s.F && T >= 4) ? NX_PATH_MFMA_SPLIT : NX_PATH_GEMV;
+    return (tpe >= 1.8 || ((long)T * k >= 64 && tpe >= 1.2)) ? NX_PATH_MFMA_SPLIT : NX_PATH_GEMV;
+  }
+  if (split_fmt && shared && s.Fs == s.F && (large || s.fmt == NX_FMT_Q4_K)) {
+    // A shared expert sees every token: the GEMV walks it a token pair at
+    // a time, the split-activation path 16 tokens at a time.  Measured
+    // (DeepSeek shapes, us, GEMV / split / grouped GEMM): Q4_K 2 tokens 105
+    // / 128 / 233, 4: 265 / 196 / 282, 27: 9257 / 836 / 1251, 128: - / 1546 /
+    // 1989, 256 (8 per routed expert): - / 1836 / 2090, 400 (12.5): - / 2105
+    // / 2123; Q4_0 4: 232 / 198 / 281, 27: - / 950 / 1226, 128: - / 1665 /
+    // 1960; Q8_0 8: 840 / 542 / 643, 27: - / 1357
+    // / 1524, 300 (9.4): - / 2924 / 2730.
+    if (tpe >= (large && !q8 ? 12.0 : 8.0)) return NX_PATH_MFMA_BF16;
+    return T >= (q8 ? 6 : 4) ? NX_PATH_MFMA_SPLIT : NX_PATH_GEMV;
+  }
+  if (split_fmt && !shared) {
+    // The GEMV re-reads an expert's weights per pair of its tokens, the
+    // split-activation path reads them once per 16 tokens, and the grouped
+    // GEMM once, at bf16 operands.  Measured (us, GEMV / split / grouped
+    // GEMM) by tokens per expert: Mixtral Q4_0 1.1: 80 / 96 / 176, 1.5: 154 /
+    // 130 / 240, 2.0: 249 / 155 / 244; Q4_K 1.3: 128 / 107 / 201, 2.2: 454 /
+    // 156 / 254, 8: 906 / 215 / 301, 12: - / 241 / 304, 16: - / 320 / 305;
+    // Q8_0 2.0: 320 / 239 / 295, 8: - / 338 / 363, 16: - / 540 / 365; Qwen3
+    // Q4_K 1.1: 45 / 50 / 68, 1.3: 107 / 64 / 93, 8: - / 132 / 151, 12.5: -
+    // / 137 / 153, 16: - / 155 / 156.  Smaller layers (GEMV / split): 8
+    // experts of 4096 x 1792 Q4_K 1.3: 38 / 37, 1.6: 57 / 43, Q8_0 1.6: 48 /
+    // 54, 2.2: 59 / 54; 1024 x 2048 Q4_K 1.3: 31 / 35, 1.6: 42 / 35; 512 x
+    // 1024 Q4_K 1.6: 25 / 34, 2.2: 35 / 36, 3.1: 46 / 37; 64 experts of 1024
+    // x 768, top 8, 1.1: 35 / 35, 1.3: 53 / 36.
+    const long pairs = (long)T * k;
+    if (tpe >= (large && !q8 ? 13.0 : 12.0)) return NX_PATH_MFMA_BF16;
+    if (tpe >= 3.0 || (pairs >= 64 && tpe >= 1.2) || (fits && pairs >= 40 && tpe >= 1.25) ||
+        (large && tpe >= (q8 ? 2.0 : 1.28)) || (fits && !q8 && weights >= 2e6 && tpe >= 1.6))
+      return NX_PATH_MFMA_SPLIT;
+    return NX_PATH_GEMV;
+  }
+  if (s.fmt == NX_FMT_F32) {
+    // f32 weights keep their precision on the GEMV; the bf16 grouped GEMM
+    // only once experts see 32 tokens on average
+    const long active_max = std::min<long>(s.E, (long)T * k);
+    return ((long)T * k >= 32 * active_max) ? NX_PATH_MFMA_BF16 : NX_PATH_GEMV;
+  }
+  // The grouped GEMM from ~3 tokens per routed expert (Mixtral Q8_0 and
+  // Q4_0 at 8 and 16 tokens, Qwen3 Q8_0 at 32), or from 6 tokens when a
+  // shared expert sees them all: the GEMV passes over the shared expert
+  // per pair of tokens and over the routed experts per token group
+  // (DeepSeek shapes with a shared expert: GEMV 0.29 / 0.81 / 10.5 ms
+  // at 4 / 8 / 32 tokens, grouped GEMM 0.36 / 0.61 / 1.44 ms).
+  return (tpe >= 3.0 || (shared && T >= 6)) ? NX_PATH_MFMA_BF16 : NX_PATH_GEMV;
+}
+
+}  // namespace nx

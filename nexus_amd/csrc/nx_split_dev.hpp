@@ -142,7 +142,8 @@ __device__ __forceinline__ float split16(const f32x4 (&v)[4], int j16, Put put, 
 // at 16 ((2 u + (hi 0, lo 1)) 4 + g) + 2 p, so the four lane groups of a row
 // read 64 contiguous bytes; then the min term's operands (8 bytes per lane
 // group in Q4_K, 16 in Q2_K) and the unscale factor.
-constexpr int REC_XM = 1024, REC_SX = 1088, REC_BYTES = 1152;
+constexpr int REC_XM = 1024, REC_SX = 1088;
+static_assert(REC_SX + 64 == REC_BYTES, "a record is whole 128-byte lines");
 
 // the record of one (row, chunk), written by its 16 lanes
 template <int FMT>

@@ -1,0 +1,54 @@
+"""What a MoE call's sizes decide (nexus_amd/csrc/nx_plan.hpp): the path AUTO
+takes and the split-activation path's workspace.  CPU only: the header is plain
+C++ and is compiled on its own with the host compiler.
+"""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "nexus_amd", "csrc")
+GXX = shutil.which("g++")
+
+pytestmark = pytest.mark.skipif(GXX is None, reason="no host C++ compiler")
+
+
+def run(tmp_path, body):
+    """Compiles `body` as main()'s statements over the header and runs it."""
+    src, exe = tmp_path / "check.cpp", tmp_path / "check"
+    src.write_text('#include <cstdio>\n#include "nx_plan.hpp"\nusing namespace nx;\n'
+                   "int main() {\n  int bad = 0;\n" + body + "\n  return bad ? 1 : 0;\n}\n")
+    r = subprocess.run([GXX, "-std=c++17", "-O1", "-Wall", "-Werror", f"-I{CSRC}", str(src), "-o", str(exe)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, f"exit {r.returncode}\n{r.stdout[-2000:]}"
+    return r.stdout
+
+
+def test_any_width_has_a_path_in_the_scratch_array(tmp_path):
+    """Every format and width that an expert set may have gets a path, with and
+    without a limit on the workspace; a layer that is not in whole 256-weight
+    chunks (narrower than one among them) never the split path."""
+    run(tmp_path, r"""
+  const int fmts[] = {NX_FMT_F32, NX_FMT_F16, NX_FMT_BF16, NX_FMT_Q4_0, NX_FMT_Q8_0, NX_FMT_Q4_K, NX_FMT_Q2_K};
+  for (int fmt : fmts)
+    for (int H : {1, 32, 96, 128, 224, 256, 288, 512, 4096})
+      for (int F : {1, 32, 96, 128, 224, 256, 288, 512, 14336})
+        for (int Fs : {0, 32, F})
+          for (int T : {1, 2, 3, 5, 8, 33, 1000})
+            for (int k : {1, 2, 8})
+              for (size_t scratch : {(size_t)64 << 20, SIZE_MAX}) {
+                const bool super = fmt == NX_FMT_Q4_K || fmt == NX_FMT_Q2_K;
+                if (super && (H % 256 || F % 256)) continue;  // refused when created
+                const int p = auto_path({fmt, 8, H, F, Fs}, T, k, scratch);
+                const bool chunks = H % 256 == 0 && F % 256 == 0 && fmt != NX_FMT_F32 &&
+                                    fmt != NX_FMT_F16 && fmt != NX_FMT_BF16;
+                if (p == NX_PATH_AUTO || (p == NX_PATH_MFMA_SPLIT && !chunks)) {
+                  std::printf("fmt %d H %d F %d Fs %d T %d k %d: path %d\n", fmt, H, F, Fs, T, k, p);
+                  ++bad;
+                }
+              }
+""")

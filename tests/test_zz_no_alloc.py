@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 
 import nexus_amd as nx
-from moe_cases import Q2_K, Q4_0, Q4_K, Q8_0, DeviceArray, Layer, assert_same_bits
+from moe_cases import F32, Q2_K, Q4_0, Q4_K, Q8_0, DeviceArray, Layer, assert_same_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -53,6 +53,11 @@ CASES = [
     (Q8_0, 8, 512, 1024, 2, 0, 0, nx.PATH_MFMA_SPLIT, (24, 5)),
     (Q2_K, 8, 512, 1024, 2, 0, 0, nx.PATH_MFMA_SPLIT, (24, 5)),
     (Q2_K, 16, 512, 512, 4, 512, 1, nx.PATH_MFMA_SPLIT, (12, 4)),
+    # widths of less than one 256-weight chunk: never the split path
+    (Q8_0, 8, 128, 512, 2, 0, 0, nx.PATH_AUTO, (40, 3)),
+    (Q4_0, 8, 512, 96, 2, 0, 0, nx.PATH_AUTO, (16, 1)),
+    (Q8_0, 8, 256, 128, 2, 128, 1, nx.PATH_AUTO, (9, 2)),
+    (F32, 8, 64, 96, 2, 0, 0, nx.PATH_AUTO, (12, 1)),
 ]
 
 
