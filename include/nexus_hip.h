@@ -90,8 +90,8 @@ extern "C" {
 #define NX_PATH_AUTO 0      /* by tokens per expert and the layer's size: GEMV, then (Q4_K and
                                Q2_K, and Q4_0 and Q8_0 in whole 256-weight chunks; with no
                                shared expert or one as wide as the routed experts, Q4_0 and
-                               Q8_0 there only in large layers) the split-activation MFMA
-                               path, then (not Q2_K) the grouped GEMM on bf16 operands */
+                               Q8_0 there only in large layers; x 16-byte aligned) the
+                               split-activation MFMA path, then (not Q2_K) the grouped GEMM on bf16 operands */
 #define NX_PATH_GEMV 1      /* dequant-in-register GEMV, fp32 accumulate */
 #define NX_PATH_MFMA_F16 2  /* grouped GEMM on fp16 MFMA, fp32 accumulate; activations and
                                SwiGLU outputs must stay within fp16's range (|v| < 65504) */
@@ -101,7 +101,8 @@ extern "C" {
                                 on the raw codes with activations split into two fp16 halves,
                                 block and sub-block scales applied to the products; no
                                 dequantization.  A shared expert must have the routed experts'
-                                ff_dim */
+                                ff_dim, and x must be 16-byte aligned (other paths: any float
+                                address) */
 
 /* expert matrix roles */
 #define NX_ROLE_GATE 0 /* [ff_dim x hidden] */

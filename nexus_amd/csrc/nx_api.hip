@@ -957,7 +957,8 @@ int nx::moe_forward(nx_ctx *c, const nx_experts *ex, const float *d_x, const flo
                 "Q2_K experts run on the GEMV and the split-activation MFMA path only");
   }
   if (use == NX_PATH_AUTO)
-    use = auto_path(shape_of(ex), T, k, c->scratch_mode ? kScratchBytes : SIZE_MAX);
+    use = auto_path(shape_of(ex), T, k, (reinterpret_cast<uintptr_t>(d_x) & 15) == 0,
+                    c->scratch_mode ? kScratchBytes : SIZE_MAX);
 
   if (use == NX_PATH_GEMV) {
     NX_TRY(ws(c, WS_YPAIR, pairs_total * H, &d_ypair));

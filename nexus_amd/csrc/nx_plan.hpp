@@ -69,13 +69,14 @@ inline size_t mfv_bytes(const MoeShape &s, int T, int k) {
 }
 
 // ---- AUTO
-// The path of a call on T tokens, top k.  scratch: the bytes its workspace may
+// The path of a call on T tokens, top k.  aligned: x on 16 bytes, which the
+// split path needs and the others do not.  scratch: the bytes its workspace may
 // take (SIZE_MAX where it is allocated).
 //
 // AUTO takes bf16 operands on the grouped GEMM: fp16's range ends at 65504,
 // which SwiGLU activations of real models can pass; bf16 keeps float32's range,
 // runs as fast here, and stays within the MFMA bar.
-inline int auto_path(const MoeShape &s, int T, int k, size_t scratch) {
+inline int auto_path(const MoeShape &s, int T, int k, bool aligned, size_t scratch) {
   if (s.fmt == NX_FMT_F16 || s.fmt == NX_FMT_BF16) return NX_PATH_GEMV;
   const bool shared = s.Fs > 0;
   // Tokens per active expert, with the active count expected under
@@ -89,7 +90,7 @@ inline int auto_path(const MoeShape &s, int T, int k, size_t scratch) {
   // In the fixed scratch array of nx_moe_forward_noalloc a batch that its
   // workspace would not fit keeps the narrower ranges, whose other paths
   // need less.
-  const bool split_fmt = mfv_supports(s);
+  const bool split_fmt = aligned && mfv_supports(s);
   const bool fits = split_fmt && (scratch == SIZE_MAX || mfv_bytes(s, T, k) + (size_t)T * k * 64 +
                                                                  (size_t)s.E * 64 + (1u << 20) <=
                                                              scratch);
@@ -103,6 +104,7 @@ inline int auto_path(const MoeShape &s, int T, int k, size_t scratch) {
     // 0.534; Qwen3 4 tokens 0.048 / 0.048, 8: 0.093 / 0.065, 512: 1.84 /
     // 0.265; DeepSeek with its shared expert 2 tokens 0.119 / 0.137, 4:
     // 0.307 / 0.218, 64: 44.1 / 1.52.
+    if (!split_fmt) return NX_PATH_GEMV;
     if (shared) return (s.Fs == s.F && T >= 4) ? NX_PATH_MFMA_SPLIT : NX_PATH_GEMV;
     return (tpe >= 1.8 || ((long)T * k >= 64 && tpe >= 1.2)) ? NX_PATH_MFMA_SPLIT : NX_PATH_GEMV;
   }

@@ -43,7 +43,7 @@ def test_any_width_has_a_path_in_the_scratch_array(tmp_path):
               for (size_t scratch : {(size_t)64 << 20, SIZE_MAX}) {
                 const bool super = fmt == NX_FMT_Q4_K || fmt == NX_FMT_Q2_K;
                 if (super && (H % 256 || F % 256)) continue;  // refused when created
-                const int p = auto_path({fmt, 8, H, F, Fs}, T, k, scratch);
+                const int p = auto_path({fmt, 8, H, F, Fs}, T, k, true, scratch);
                 const bool chunks = H % 256 == 0 && F % 256 == 0 && fmt != NX_FMT_F32 &&
                                     fmt != NX_FMT_F16 && fmt != NX_FMT_BF16;
                 if (p == NX_PATH_AUTO || (p == NX_PATH_MFMA_SPLIT && !chunks)) {
@@ -51,4 +51,27 @@ def test_any_width_has_a_path_in_the_scratch_array(tmp_path):
                   ++bad;
                 }
               }
+""")
+
+
+def test_unaligned_inputs_stay_off_the_split_path(tmp_path):
+    """The split path reads x in 16-byte runs.  Calls on other addresses take
+    the rule of the formats without it: the grouped GEMM (Q2_K: none) from 3
+    tokens per expert or 6 with a shared expert, the GEMV below."""
+    run(tmp_path, r"""
+  for (int fmt : {NX_FMT_Q4_0, NX_FMT_Q8_0, NX_FMT_Q4_K, NX_FMT_Q2_K})
+    for (int H : {256, 1024, 4096})
+      for (int F : {256, 2048, 14336})
+        for (int Fs : {0, 32 * 8, F})
+          for (int T = 1; T < 400; ++T)
+            for (size_t scratch : {(size_t)64 << 20, SIZE_MAX}) {
+              const double tpe = T * 2 / (8 * (1.0 - std::pow(0.75, (double)T)));
+              const int want = fmt != NX_FMT_Q2_K && (tpe >= 3.0 || (Fs && T >= 6)) ? NX_PATH_MFMA_BF16
+                                                                                    : NX_PATH_GEMV;
+              const int p = auto_path({fmt, 8, H, F, Fs}, T, 2, false, scratch);
+              if (p != want) {
+                std::printf("fmt %d H %d F %d Fs %d T %d: path %d\n", fmt, H, F, Fs, T, p);
+                ++bad;
+              }
+            }
 """)
