@@ -165,7 +165,7 @@ enum WsSlot {
   WS_BLK_HIDDEN,
   WS_MAT_X,    // device copy of matvec inputs for blocking calls
   WS_MAT_Y,
-  WS_MFV_PART, // gate/up partial sums of the split-activation MFMA path
+  WS_MFV_PART, // partial sums and records of the split-activation MFMA path
   WS_TILES_DOWN, // grouped-GEMM tile list of the down pass
   WS_PERM_CHUNK, // per-chunk expert counts of the many-workgroup permutation
   WS_COUNT

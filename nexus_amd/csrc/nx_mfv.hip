@@ -399,11 +399,10 @@ int run_mfv(nx_ctx *c, const MfvPlan &p) {
   const MfvSizes z = mfv_sizes(shape_of(ex), p.T, p.k);
   const size_t pairs = z.pairs;
   const int nks_g = z.nks_g, nks_d = z.nks_d;
-  void *vp, *vr;
-  NX_TRY(ws_get(c, WS_MFV_PART, z.part, &vp));
-  NX_TRY(ws_get(c, WS_ACT, z.recs, &vr));
+  void *vp;
+  NX_TRY(ws_get(c, WS_MFV_PART, z.bytes, &vp));
   float *ppart = static_cast<float *>(vp);
-  uint8_t *rec = static_cast<uint8_t *>(vr);
+  uint8_t *rec = static_cast<uint8_t *>(vp) + z.act_at;
   for (int pass = 0; pass < 2; ++pass) {
     const bool gateup = pass == 0;
     const RolePlane &R0 = ex->role[gateup ? NX_ROLE_GATE : NX_ROLE_DOWN];
@@ -472,8 +471,8 @@ int mfv_max_tiles(int T, int k, int E, bool shared) {
 int mfv_records(nx_ctx *c, const nx_experts *ex, int T, int k, uint8_t **rec) {
   const MfvSizes z = mfv_sizes(shape_of(ex), T, k);
   void *p;
-  NX_TRY(ws_get(c, WS_MFV_PART, z.part, &p));
-  *rec = static_cast<uint8_t *>(p) + z.gate;
+  NX_TRY(ws_get(c, WS_MFV_PART, z.bytes, &p));
+  *rec = static_cast<uint8_t *>(p) + z.x_at;
   return NX_OK;
 }
 

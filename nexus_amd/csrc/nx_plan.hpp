@@ -38,12 +38,15 @@ inline int mv_slice_chunks(int nchunk) {
   return (nchunk + n - 1) / n;
 }
 
-// Both passes' partial sums share one buffer: the down pass writes it after
-// the gate/up sums, and x's records behind them, are dead.
+// The path's workspace is one buffer.  At its start lie the gate/up sums, then
+// the down sums; x's records follow the gate/up sums, and the gated rows'
+// records end the buffer.  The SwiGLU kernel writes those when x's records are
+// dead, the down pass its sums when the gate/up sums are, so each pair that is
+// in use at one time lies apart.
 struct MfvSizes {
   size_t pairs;
   int ks_g, ks_d, nks_g, nks_d;  // chunks per K slice, slices
-  size_t gate, part, recs;       // bytes: gate/up sums, the shared buffer, the gated rows' records
+  size_t x_at, act_at, bytes;    // offsets of x's and the gated rows' records; the buffer
 };
 
 inline MfvSizes mfv_sizes(const MoeShape &s, int T, int k) {
@@ -56,17 +59,17 @@ inline MfvSizes mfv_sizes(const MoeShape &s, int T, int k) {
   z.ks_d = mv_slice_chunks(cd);
   z.nks_g = (cg + z.ks_g - 1) / z.ks_g;
   z.nks_d = (cd + z.ks_d - 1) / z.ks_d;
-  z.gate = (size_t)z.nks_g * pairs * 2 * s.F * sizeof(float);
-  z.part = std::max(z.gate + (size_t)T * cg * REC_BYTES, (size_t)z.nks_d * pairs * s.H * sizeof(float));
-  z.recs = pairs * cd * REC_BYTES;
+  const size_t gate = (size_t)z.nks_g * pairs * 2 * s.F * sizeof(float);
+  const size_t down = (size_t)z.nks_d * pairs * s.H * sizeof(float);
+  const size_t xrec = (size_t)T * cg * REC_BYTES, arec = pairs * cd * REC_BYTES;
+  z.x_at = gate;
+  z.bytes = std::max({gate + xrec, gate + arec, down + arec});
+  z.act_at = z.bytes - arec;
   return z;
 }
 
 // its workspace, but the routes'
-inline size_t mfv_bytes(const MoeShape &s, int T, int k) {
-  const MfvSizes z = mfv_sizes(s, T, k);
-  return z.part + z.recs;
-}
+inline size_t mfv_bytes(const MoeShape &s, int T, int k) { return mfv_sizes(s, T, k).bytes; }
 
 // ---- AUTO
 // The path of a call on T tokens, top k.  aligned: x on 16 bytes, which the

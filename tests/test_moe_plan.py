@@ -75,3 +75,35 @@ def test_unaligned_inputs_stay_off_the_split_path(tmp_path):
               }
             }
 """)
+
+
+def test_split_workspace(tmp_path):
+    """The split path's buffer: x's records apart from the gate/up sums, the
+    gated rows' records apart from both passes' sums, all inside it and on
+    128-byte lines.  It is never larger than f32 gated rows and the sums of both
+    passes side by side, in K slices of 4 and 3 chunks: a call of the
+    no-allocation entry point that fitted with those still does."""
+    run(tmp_path, r"""
+  for (int cg = 1; cg <= 64; ++cg)
+    for (int cd = 1; cd <= 112; ++cd)
+      for (int k : {1, 2, 4, 8})
+        for (int shared = 0; shared < 2; ++shared)
+          for (int T : {1, 3, 17, 4099}) {
+            const MoeShape s{NX_FMT_Q4_K, 64, 256 * cg, 256 * cd, shared ? 256 * cd : 0};
+            const MfvSizes z = mfv_sizes(s, T, k);
+            const size_t p = z.pairs, f = sizeof(float);
+            const size_t gate = z.nks_g * p * 2 * s.F * f, down = z.nks_d * p * s.H * f;
+            const size_t xrec = (size_t)T * cg * REC_BYTES, arec = p * cd * REC_BYTES;
+            const size_t most = ((cg + 3) / 4 * 2 * s.F + s.F + (size_t)((cd + 2) / 3) * s.H) * p * f;
+            bool ok = p == (size_t)T * (k + shared) && z.ks_g >= 1 && z.ks_g <= MV_KW && z.ks_d >= 1 &&
+                      z.ks_d <= MV_KW && z.nks_g * z.ks_g >= cg && (z.nks_g - 1) * z.ks_g < cg &&
+                      z.nks_d * z.ks_d >= cd && (z.nks_d - 1) * z.ks_d < cd;
+            ok = ok && z.x_at >= gate && z.x_at + xrec <= z.bytes && z.act_at >= gate && z.act_at >= down &&
+                 z.act_at + arec <= z.bytes && z.x_at % 128 == 0 && z.act_at % 128 == 0 && z.bytes <= most;
+            if (!ok) {
+              std::printf("cg %d cd %d k %d shared %d T %d: %zu bytes, at most %zu\n", cg, cd, k, shared, T,
+                          z.bytes, most);
+              ++bad;
+            }
+          }
+""")

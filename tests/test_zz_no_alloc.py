@@ -53,6 +53,8 @@ CASES = [
     (Q8_0, 8, 512, 1024, 2, 0, 0, nx.PATH_MFMA_SPLIT, (24, 5)),
     (Q2_K, 8, 512, 1024, 2, 0, 0, nx.PATH_MFMA_SPLIT, (24, 5)),
     (Q2_K, 16, 512, 512, 4, 512, 1, nx.PATH_MFMA_SPLIT, (12, 4)),
+    # nearly all of the scratch array
+    (Q8_0, 8, 256, 512, 1, 0, 0, nx.PATH_MFMA_SPLIT, (9300, 77)),
     # widths of less than one 256-weight chunk: never the split path
     (Q8_0, 8, 128, 512, 2, 0, 0, nx.PATH_AUTO, (40, 3)),
     (Q4_0, 8, 512, 96, 2, 0, 0, nx.PATH_AUTO, (16, 1)),
