@@ -45,7 +45,7 @@
 // arithmetic alone 99.  Against workgroups of 256 rows that staged their
 // activations in LDS and walked a slice of 4 chunks (us, layer): Mixtral 32
 // tokens 247 -> 211, DeepSeek 27 tokens 1008 -> 806, Qwen3 61 tokens 118.6 ->
-// 113.9; error against 64 bits 9.3e-7 -> 3.9e-7 (Q4_K), 7.8e-5 -> 2.1e-7 (Q4_0,
+// 108; error against 64 bits 9.3e-7 -> 3.9e-7 (Q4_K), 7.8e-5 -> 2.1e-7 (Q4_0,
 // whose codes were fp16 subnormals).  A wave per 64 rows that walked the chunks
 // itself read each line's halves a chunk apart, too late for the L2: 370 us.
 #include "nx_internal.hpp"
@@ -89,8 +89,8 @@ struct MfvStep {
   u32x4_t m;
 };
 
-constexpr int MV_STEPS = 8;  // (row tile, matrix) steps per pass of the loop
-constexpr int MV_D = 4;      // steps in flight (2, 3 or 6: within 3%)
+constexpr int MV_STEPS = 4;  // (row tile, matrix) steps per pass of the loop
+constexpr int MV_D = 4;      // steps in flight, at most MV_STEPS (2, 3 or 6: within 3%)
 
 template <bool GATEUP, int FMT>
 __global__ __launch_bounds__(64 * MV_KW, 2) void k_mfv(const MfvArgs a) {
@@ -98,20 +98,25 @@ __global__ __launch_bounds__(64 * MV_KW, 2) void k_mfv(const MfvArgs a) {
   constexpr bool BLK = !Q4K && !Q2K;  // one MFMA per 32-weight block
   constexpr int D = MV_D, NQ = MfvStep<FMT>::NQ;
   constexpr int RT = GATEUP ? MV_STEPS / 2 : MV_STEPS;  // row tiles per pass
-  extern __shared__ f32x4 red[];  // [half pass][wave][step of the half][lane]
+  extern __shared__ f32x4 red[];  // [pass parity][wave][step][lane]
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // The work is a line of (tile, slice, pass of RT row tiles), each workgroup
+  // The work is a line of (tile, slice, pass of RT row tiles); each workgroup
   // takes an equal run of it.  (Workgroups of a fixed run of rows, sized on the
   // host from the expected tile count, left CUs idle wherever the routing
-  // drew another: Mixtral 32 tokens 223 us, Qwen3 61 tokens 135 us.)
+  // drew another: Mixtral 32 tokens 223 us, Qwen3 61 tokens 135 us.)  Passes are
+  // as short as the steps in flight allow, and few segments are not shared out
+  // across their ends (mfv_run): a run of one or two passes more than the
+  // others' is the round's tail.  Equal runs of 8-step passes took (layer, 8
+  // experts, top 2) 1024 x 2048 Q8_0 256 tokens 97 us, now 75; 2048 x 1280 Q4_K
+  // 128 tokens 68, now 56.
   const int ntile = a.tiles[0], npass = (a.rows >> 4) / RT;
-  const long work = (long)ntile * a.nks * npass;
-  const long u1 = work * (blockIdx.x + 1) / gridDim.x;
-  for (long un = work * blockIdx.x / gridDim.x; un < u1;) {
+  const MfvRun run = mfv_run((int)blockIdx.x, (int)gridDim.x, ntile * a.nks, npass);
+  int buf = 0;  // the sums' buffer of this pass: red + 0 or + ks MV_STEPS 64
+  for (long un = run.u0; un < run.u1;) {
     const int seg = (int)(un / npass), pass0 = (int)(un - (long)seg * npass);
-    const int pass1 = (int)min((long)npass, pass0 + (u1 - un));
+    const int pass1 = (int)min((long)npass, pass0 + (run.u1 - un));
     un += pass1 - pass0;
     const int tile = seg / a.nks, slice = seg - tile * a.nks;
     // tile t: expert tiles[2 + 2t] (E: the shared expert), first pair
@@ -318,31 +323,28 @@ __global__ __launch_bounds__(64 * MV_KW, 2) void k_mfv(const MfvArgs a) {
         __builtin_amdgcn_sched_barrier(0);
         issue(ring[(i + D) % MV_STEPS], i + D < MV_STEPS ? rt : rt + RT, (i + D) % MV_STEPS);
         __builtin_amdgcn_sched_barrier(0);
-        // The slice's sums: every half pass the waves leave their chunks' results
-        // in one of two buffers, and wave w adds those of steps w, w + ks, ... in
-        // chunk order.  One barrier per half pass: a buffer is written again
-        // only after the next half pass's barrier.
-        constexpr int HALF = MV_STEPS / 2;
-        f32x4 *half = red + i / HALF * a.ks * HALF * 64 + lane;
-        half[(wave * HALF + i % HALF) * 64] = res;
-        if (i % HALF == HALF - 1) {
-          __syncthreads();
-          for (int t = wave; t < HALF; t += a.ks) {
-            f32x4 sum = half[t * 64];
-            for (int v = 1; v < a.ks; ++v) {
-              const f32x4 r = half[(v * HALF + t) * 64];
-#pragma unroll
-              for (int k = 0; k < 4; ++k) sum[k] += r[k];
-            }
-            // lane holds row (lane % 16), pairs 4g .. 4g+3
-            const int st = i / HALF * HALF + t;
-            float *o = out + (GATEUP ? 16 * (rt + (st >> 1)) + (st & 1) * a.rows : 16 * (rt + st));
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-              if (4 * g + k < cnt) o[(size_t)k * a.out_stride] = sum[k];
-          }
-        }
+        red[buf + (wave * MV_STEPS + i) * 64 + lane] = res;
       }
+      // The slice's sums: every pass the waves leave their chunks' results in one
+      // of two buffers, and wave w adds those of steps w, w + ks, ... in chunk
+      // order.  One barrier per pass: a buffer is written again only after the
+      // next pass's barrier.
+      __syncthreads();
+      for (int t = wave; t < MV_STEPS; t += a.ks) {
+        const f32x4 *r = red + buf + t * 64 + lane;
+        f32x4 sum = *r;
+        for (int v = 1; v < a.ks; ++v) {
+          r += MV_STEPS * 64;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) sum[k] += (*r)[k];
+        }
+        // lane holds row (lane % 16), pairs 4g .. 4g+3
+        float *o = out + (GATEUP ? 16 * (rt + (t >> 1)) + (t & 1) * a.rows : 16 * (rt + t));
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (4 * g + k < cnt) o[(size_t)k * a.out_stride] = sum[k];
+      }
+      buf ^= a.ks * MV_STEPS * 64;
     }
   }
 }
@@ -439,9 +441,12 @@ int run_mfv(nx_ctx *c, const MfvPlan &p) {
     a.out_split = pairs * a.out_stride;
     a.ks = gateup ? z.ks_g : z.ks_d;
     a.nks = gateup ? nks_g : nks_d;
-    // one round of resident workgroups: 8 waves per CU (registers)
+    // At most 8 waves per CU.  Registers allow 12 (Q8_0: 8), but with as many
+    // workgroups as fit the layers whose slices leave room got slower: 32 experts
+    // of 2560 x 1536, top 4, Q2_K 12 tokens 63 -> 77 us; 16 of 4096 x 2304, top
+    // 4, Q4_K 6 tokens 76 -> 84 us.
     const dim3 grid((unsigned)(c->num_cu * (MV_KW / a.ks))), block(64 * a.ks);
-    const uint32_t lds = 2 * a.ks * (MV_STEPS / 2) * 64 * sizeof(f32x4);
+    const uint32_t lds = 2 * a.ks * MV_STEPS * 64 * sizeof(f32x4);
     if (gateup) {
       NX_TRY(launch(c, "mfv_gateup", [&] { go(c, k_mfv<true, FMT>, grid, block, lds, a); }));
       const size_t n = pairs * cd;

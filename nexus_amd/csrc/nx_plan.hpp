@@ -71,6 +71,29 @@ inline MfvSizes mfv_sizes(const MoeShape &s, int T, int k) {
 // its workspace, but the routes'
 inline size_t mfv_bytes(const MoeShape &s, int T, int k) { return mfv_sizes(s, T, k).bytes; }
 
+// A workgroup's run of k_mfv's work: units [u0, u1) of a line of nseg segments
+// (a tile's K slice) of npass passes each.  Where the segments are fewer than
+// the workgroups, each gets its own ones: a run that crosses into another
+// segment waits a second time for the chain of loads that finds the pairs, about
+// two passes' time.  Otherwise, or where whole segments leave some workgroups
+// more than that much extra, the line is cut into equal runs.
+struct MfvRun {
+  long u0, u1;
+};
+constexpr MfvRun mfv_run(int block, int nblocks, int nseg, int npass) {
+  if (nseg <= 0) return {0, 0};
+  const long work = (long)nseg * npass;
+  const int least = nblocks / nseg;  // workgroups of a segment, at least
+  if (least > 0 && (npass + least - 1) / least <= (work + nblocks - 1) / nblocks + 2) {
+    const int seg = (int)((long)block * nseg / nblocks);
+    const int b0 = (int)(((long)seg * nblocks + nseg - 1) / nseg);
+    const int n = (int)(((long)(seg + 1) * nblocks + nseg - 1) / nseg) - b0;
+    const long at = (long)seg * npass;
+    return {at + (long)npass * (block - b0) / n, at + (long)npass * (block - b0 + 1) / n};
+  }
+  return {work * block / nblocks, work * (block + 1) / nblocks};
+}
+
 // ---- AUTO
 // The path of a call on T tokens, top k.  aligned: x on 16 bytes, which the
 // split path needs and the others do not.  scratch: the bytes its workspace may

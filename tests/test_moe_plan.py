@@ -107,3 +107,26 @@ def test_split_workspace(tmp_path):
             }
           }
 """)
+
+
+def test_split_runs_cover_the_line_once(tmp_path):
+    """The workgroups' runs of the split kernel follow each other over the whole
+    line, each unit once, and none is longer than an equal share and two passes."""
+    run(tmp_path, r"""
+  for (int nb : {256, 512, 304, 1})
+    for (int nseg = 0; nseg <= 700; nseg += nseg < 40 ? 1 : 13)
+      for (int npass : {2, 4, 5, 8, 20, 32, 64, 112, 448}) {
+        long at = 0, most = 0;
+        for (int b = 0; b < nb; ++b) {
+          const MfvRun r = mfv_run(b, nb, nseg, npass);
+          if (r.u0 != at || r.u1 < r.u0) ++bad;
+          at = r.u1;
+          most = std::max(most, r.u1 - r.u0);
+        }
+        const long work = (long)nseg * npass;
+        if (at != work || most > (work + nb - 1) / nb + 2) {
+          std::printf("%d workgroups, %d segments of %d: %ld of %ld, at most %ld\n", nb, nseg, npass, at, work, most);
+          ++bad;
+        }
+      }
+""")
