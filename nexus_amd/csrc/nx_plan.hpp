@@ -160,10 +160,22 @@ inline int auto_path(const MoeShape &s, int T, int k, bool aligned, size_t scrat
     // 54, 2.2: 59 / 54; 1024 x 2048 Q4_K 1.3: 31 / 35, 1.6: 42 / 35; 512 x
     // 1024 Q4_K 1.6: 25 / 34, 2.2: 35 / 36, 3.1: 46 / 37; 64 experts of 1024
     // x 768, top 8, 1.1: 35 / 35, 1.3: 53 / 36.
+    // The GEMV's time hangs on how the tokens pair up, so the lower limits are
+    // from means over eight routings (GEMV / split): large layers Q4_K 1.3:
+    // Mixtral 136 / 113, 16 experts of 4096 x 2304 61 / 57; Q4_0 1.3: 102 / 117
+    // and 51 / 61, 1.46: 138 / 132 and 69 / 65; Q8_0 2.0: 286 / 255 and 136 /
+    // 110.  Of 7 M weights: 4 experts of 2048 x 3584 Q4_K 6 pairs 34 / 36, 8
+    // pairs 40 / 37, Q8_0 10 pairs 42 / 43; 8 of 4096 x 1792 Q4_K 6 pairs 37 /
+    // 40, 8 pairs 46 / 43, Q8_0 14 pairs 52 / 56, 16 pairs 61 / 57.  64 of 1024
+    // x 768 Q8_0 1.28: 38 / 42, 1.36: 49 / 45.
     const long pairs = (long)T * k;
     if (tpe >= (large && !q8 ? 13.0 : 12.0)) return NX_PATH_MFMA_BF16;
-    if (tpe >= 3.0 || (pairs >= 64 && tpe >= 1.2) || (fits && pairs >= 40 && tpe >= 1.25) ||
-        (large && tpe >= (q8 ? 2.0 : 1.28)) || (fits && !q8 && weights >= 2e6 && tpe >= 1.6))
+    // the least tokens per expert of a large layer; the smallest of them with a
+    // few pairs are bound by the launches, of which the GEMV has fewer
+    const double least = q8 ? 2.0 : s.fmt == NX_FMT_Q4_0 ? 1.4 : 1.28;
+    const bool few = weights < 9e6 && pairs < (q8 ? 16 : 8);
+    if (tpe >= 3.0 || (pairs >= 64 && tpe >= 1.2) || (fits && pairs >= 40 && tpe >= (q8 ? 1.3 : 1.25)) ||
+        (large && !few && tpe >= least) || (fits && !q8 && !few && weights >= 2e6 && tpe >= 1.6))
       return NX_PATH_MFMA_SPLIT;
     return NX_PATH_GEMV;
   }

@@ -83,3 +83,46 @@ def test_unaligned_input(ctx, case):
             forward(ex.forward_dev, T, E, H, k, SPLIT, shift)
         assert e.value.code == nx.NX_ERR_UNSUPPORTED
     ex.close()
+
+
+# fmt, E, H, F, k, shared F, T, path: both sides of the limits of the rule
+# (nexus_amd/csrc/nx_plan.hpp)
+CHOICE = [
+    (Q4_K, 8, 2048, 4608, 2, 0, 2, GEMV), (Q4_K, 8, 2048, 4608, 2, 0, 3, SPLIT),
+    (Q4_K, 8, 2048, 4608, 2, 0, 51, SPLIT), (Q4_K, 8, 2048, 4608, 2, 0, 53, BF16),
+    (Q4_0, 8, 2048, 4608, 2, 0, 3, GEMV), (Q4_0, 8, 2048, 4608, 2, 0, 4, SPLIT),
+    (Q4_0, 8, 2048, 4608, 2, 0, 51, SPLIT), (Q4_0, 8, 2048, 4608, 2, 0, 53, BF16),
+    (Q8_0, 8, 2048, 4608, 2, 0, 6, GEMV), (Q8_0, 8, 2048, 4608, 2, 0, 7, SPLIT),
+    (Q8_0, 8, 2048, 4608, 2, 0, 47, SPLIT), (Q8_0, 8, 2048, 4608, 2, 0, 49, BF16),
+    (Q4_0, 8, 2048, 4608, 2, 4608, 3, GEMV), (Q4_0, 8, 2048, 4608, 2, 4608, 4, SPLIT),
+    (Q4_0, 8, 2048, 4608, 2, 4608, 47, SPLIT), (Q4_0, 8, 2048, 4608, 2, 4608, 49, BF16),
+    (Q8_0, 8, 2048, 4608, 2, 4608, 5, GEMV), (Q8_0, 8, 2048, 4608, 2, 4608, 6, SPLIT),
+    (Q8_0, 8, 2048, 4608, 2, 4608, 31, SPLIT), (Q8_0, 8, 2048, 4608, 2, 4608, 33, BF16),
+    (Q4_K, 8, 1024, 2048, 2, 0, 4, GEMV), (Q4_K, 8, 1024, 2048, 2, 0, 5, SPLIT),
+    (Q8_0, 64, 1024, 768, 8, 0, 5, GEMV), (Q8_0, 64, 1024, 768, 8, 0, 6, SPLIT),
+]
+
+
+@pytest.mark.parametrize("case", CHOICE, ids=lambda c: "-".join(map(str, c)))
+def test_choice(ctx, case):
+    fmt, E, H, F, k, Fs, T, want = case
+    print("auto choice", nx.FORMAT_NAMES[fmt], case, flush=True)
+    ex = device_experts(ctx, fmt, E, H, F, Fs)
+    outs = {p: forward(ex.forward_dev, T, E, H, k, p) for p in (GEMV, SPLIT, BF16)}
+    assert_same_bits(forward(ex.forward_dev, T, E, H, k, nx.PATH_AUTO), outs[want])
+    for p, out in outs.items():  # the bits tell the paths apart
+        assert p == want or not np.array_equal(out, outs[want])
+    ex.close()
+
+
+def test_choice_in_the_scratch_array(ctx):
+    """12.6 tokens per expert, whose split workspace is above the scratch array:
+    the no-allocation call runs on the grouped GEMM, which fits."""
+    E, H, F, k, T = 64, 2304, 4096, 8, 101
+    print("auto choice, no allocation", E, H, F, k, T, flush=True)
+    ex = device_experts(ctx, Q4_K, E, H, F, 0)
+    assert_same_bits(forward(ex.forward_noalloc, T, E, H, k, nx.PATH_AUTO),
+                     forward(ex.forward_dev, T, E, H, k, BF16))
+    assert_same_bits(forward(ex.forward_dev, T, E, H, k, nx.PATH_AUTO),
+                     forward(ex.forward_dev, T, E, H, k, SPLIT))
+    ex.close()

@@ -130,3 +130,64 @@ def test_split_runs_cover_the_line_once(tmp_path):
         }
       }
 """)
+
+
+# fmt, E, H, F, shared F, top k, token counts at which AUTO's path changes:
+# the GEMV below the first, the split path from it, the grouped GEMM from the second
+AUTO_LIMITS = [
+    ("Q4_K", 8, 4096, 14336, 0, 2, 3, 52),   # 1.30 and 13 tokens per expert
+    ("Q4_0", 8, 4096, 14336, 0, 2, 4, 52),   # 1.46
+    ("Q8_0", 8, 4096, 14336, 0, 2, 7, 48),   # 2.02 and 12
+    ("Q4_0", 16, 4096, 2304, 0, 4, 4, 52),
+    ("Q8_0", 16, 4096, 2304, 0, 4, 7, 48),
+    ("Q4_K", 8, 4096, 1792, 0, 2, 4, 52),    # 7.3 M weights: from 8 pairs
+    ("Q4_K", 4, 2048, 3584, 0, 2, 4, 26),
+    ("Q4_0", 4, 2048, 3584, 0, 2, 4, 26),
+    ("Q8_0", 8, 4096, 1792, 0, 2, 8, 48),    # ... from 16 pairs
+    ("Q8_0", 4, 2048, 3584, 0, 2, 6, 24),    # ... or 3 tokens per expert
+    ("Q4_K", 8, 1024, 2048, 0, 2, 5, 48),    # 2.1 M weights: 1.64
+    ("Q8_0", 8, 1024, 2048, 0, 2, 12, 48),   # 3.1
+    ("Q4_K", 8, 512, 1024, 0, 2, 12, 48),
+    ("Q4_K", 64, 1024, 768, 0, 8, 5, 96),    # 40 pairs at 1.28
+    ("Q8_0", 64, 1024, 768, 0, 8, 6, 96),    # 1.36
+    ("Q4_K", 128, 2048, 768, 0, 8, 8, 192),  # 64 pairs
+    ("Q4_K", 256, 7168, 2048, 2048, 8, 4, 384),  # a shared expert: 4 tokens, 12 per expert
+    ("Q4_0", 256, 7168, 2048, 2048, 8, 4, 384),
+    ("Q8_0", 256, 7168, 2048, 2048, 8, 6, 256),  # 6 tokens, 8 per expert
+    ("Q4_K", 16, 512, 512, 512, 4, 4, 32),       # a small one: 8 per expert
+    ("Q4_0", 16, 512, 512, 512, 4, 6, 6),        # ... without the split path
+    ("Q4_K", 16, 512, 512, 1024, 4, 6, 6),       # a shared expert of another width
+]
+
+
+def test_auto_limits(tmp_path):
+    """Where AUTO changes its path, over 1 to 512 tokens."""
+    rows = ",".join("{{NX_FMT_%s, %d, %d, %d, %d}, %d, %d, %d}" % r for r in AUTO_LIMITS)
+    run(tmp_path, r"""
+  const struct { MoeShape s; int k, split, gemm; } rows[] = {""" + rows + r"""};
+  for (const auto &r : rows)
+    for (int T = 1; T <= 512; ++T) {
+      const int want = T < r.split ? NX_PATH_GEMV : T < r.gemm ? NX_PATH_MFMA_SPLIT : NX_PATH_MFMA_BF16;
+      const int p = auto_path(r.s, T, r.k, true, SIZE_MAX);
+      if (p != want) {
+        std::printf("fmt %d, %d experts of %d x %d, T %d: path %d\n", r.s.fmt, r.s.E, r.s.H, r.s.F, T, p);
+        ++bad;
+      }
+    }
+""")
+
+
+def test_auto_in_the_scratch_array(tmp_path):
+    """Within a limit on the workspace AUTO takes the split path over its wider
+    ranges only where that fits, and otherwise as without the wider ranges."""
+    run(tmp_path, r"""
+  const size_t limit = (size_t)64 << 20;
+  const MoeShape s{NX_FMT_Q4_K, 64, 2304, 4096, 0};
+  for (int T = 1; T <= 300; ++T) {
+    const int p = auto_path(s, T, 8, true, limit), free = auto_path(s, T, 8, true, SIZE_MAX);
+    if (mfv_bytes(s, T, 8) > limit && free == NX_PATH_MFMA_SPLIT && T * 8 >= 12 * 64 && p != NX_PATH_MFMA_BF16) ++bad;
+    if (mfv_bytes(s, T, 8) + (2u << 20) < limit && p != free) ++bad;
+  }
+  if (auto_path(s, 101, 8, true, limit) != NX_PATH_MFMA_BF16) ++bad;
+  if (auto_path(s, 101, 8, true, SIZE_MAX) != NX_PATH_MFMA_SPLIT) ++bad;
+""")
