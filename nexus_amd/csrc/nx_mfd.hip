@@ -48,9 +48,6 @@ namespace nx {
 
 namespace {
 
-constexpr int MD_K = 256;    // columns per chunk
-constexpr int MD_WAVES = 8;  // waves per workgroup
-
 struct MfdArgs {
   const uint8_t *qs, *meta;
   uint32_t qs_bytes, meta_bytes;
@@ -368,12 +365,6 @@ __global__ __launch_bounds__(64 * MD_WAVES, 2) void k_mfd(const MfdArgs a) {
   }
 }
 
-struct MfdShape {
-  int r, kw;
-  int rows() const { return 16 * r * (MD_WAVES / kw); }
-  int tokens() const { return 16 * (MD_WAVES / kw); }
-};
-
 template <int FMT>
 void (*mfd_pick(MfdShape s))(MfdArgs) {
   if (s.kw == 2) return s.r == 2 ? k_mfd<FMT, 2, 2> : k_mfd<FMT, 1, 2>;
@@ -383,13 +374,8 @@ void (*mfd_pick(MfdShape s))(MfdArgs) {
 
 }  // namespace
 
-// From five tokens: the GEMV's time grows with every two tokens, and at five it
-// is behind at every size measured (us, GEMV / MFMA: 512 x 512 Q4_K 14.2 / 5.7,
-// 1024 x 2048 Q4_0 16.7 / 5.5, 4096 x 14336 Q4_K 45 / 26, 32000 x 4096 Q8_0 70 / 40);
-// up to four tokens a call gives each token the bits of a call of its own.
 bool mfd_takes(int fmt, const RolePlane &pl, const float *x, int T) {
-  if (fmt != NX_FMT_Q4_K && fmt != NX_FMT_Q4_0 && fmt != NX_FMT_Q8_0) return false;
-  return T > 4 && pl.cols % MD_K == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
+  return mfd_sizes(fmt, pl.rows, pl.cols, T) && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
          (uint64_t)pl.rows * pl.row_qs < 0x7FFFFFF0ull;
 }
 
@@ -406,28 +392,7 @@ int launch_mfd(nx_ctx *c, int fmt, const RolePlane &pl, const float *x, int T, f
   a.T = T;
   a.x = x;
   a.out = out;
-  // One workgroup fits a CU (its stage fills the LDS), so a shape costs its
-  // rounds of the CUs times its steps of KW chunks.  Step times (us, one
-  // MI355X, all rows and tokens of a shape in use, the formats within 10%):
-  // a step costs its 8 waves about 4 us of conversion, staging and waits, and
-  // little more for more rows or token tiles, so the larger shapes win where
-  // they fill the CUs.  4096 x 4096 Q4_K, 1 x 8 / 2 x 8 / 4 x 8 / 2 x 4 / 1 x 2 /
-  // 2 x 2: 16 tokens 11.1 / 12.0 / 16.7 / 23.8 / 41.8 / 53.1 us; 64 tokens 40.3
-  // / 24.5 / 18.2 / 24.4 / 41.8 / 53.4; 509 tokens 330 / 187 / 135 / 98 / 91 /
-  // 62.
-  static const struct {
-    MfdShape s;
-    double step_us;
-  } shapes[] = {{{1, 8}, 4.0}, {{2, 8}, 4.5}, {{4, 8}, 6.8}, {{1, 4}, 4.4},
-                {{2, 4}, 5.2}, {{1, 2}, 4.8}, {{2, 2}, 6.2}};
-  MfdShape s{1, 8};
-  double best = 0.0;
-  for (const auto &t : shapes) {
-    const long wgs = (long)((pl.rows + t.s.rows() - 1) / t.s.rows()) * ((T + t.s.tokens() - 1) / t.s.tokens());
-    const double us = t.step_us * (double)((wgs + c->num_cu - 1) / c->num_cu) *
-                      (double)((a.nchunk + t.s.kw - 1) / t.s.kw);
-    if (best == 0.0 || us < best) best = us, s = t.s;
-  }
+  const MfdShape s = mfd_shape(pl.rows, a.nchunk, T, c->num_cu);
   a.ntb = (T + s.tokens() - 1) / s.tokens();
   a.nrb = (pl.rows + s.rows() - 1) / s.rows();
   const auto kern = fmt == NX_FMT_Q4_K   ? mfd_pick<NX_FMT_Q4_K>(s)

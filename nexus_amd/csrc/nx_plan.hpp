@@ -1,5 +1,5 @@
-// nx_plan.hpp — what a MoE call's sizes alone decide: the path AUTO takes and
-// the split-activation path's workspace.
+// nx_plan.hpp — what a call's sizes alone decide: the path that AUTO takes, the
+// split-activation path's workspace and runs, and the dense matvec's kernel.
 //
 // Plain C++ (no HIP): the CPU tests compile this header on its own.
 #pragma once
@@ -192,6 +192,64 @@ inline int auto_path(const MoeShape &s, int T, int k, bool aligned, size_t scrat
   // (DeepSeek shapes with a shared expert: GEMV 0.29 / 0.81 / 10.5 ms
   // at 4 / 8 / 32 tokens, grouped GEMM 0.36 / 0.61 / 1.44 ms).
   return (tpe >= 3.0 || (shared && T >= 6)) ? NX_PATH_MFMA_BF16 : NX_PATH_GEMV;
+}
+
+// ---- dense matvec on MFMA (nx_mfd.hip)
+constexpr int MD_K = 256;    // columns per chunk
+constexpr int MD_WAVES = 8;  // waves per workgroup
+
+// Whether a matrix and token count run there.  From five tokens: the GEMV's time
+// grows with every two tokens, and at five it is behind at nearly every size
+// (us, GEMV / MFMA: 512 x 512 Q4_K 14.2 / 5.7, 1024 x 2048 Q4_0 16.7 / 5.5, 4096
+// x 14336 Q4_K 45 / 26, 32000 x 4096 Q8_0 70 / 40); up to four tokens a call
+// gives each token the bits of a call of its own.  Not so where the GEMV's rows
+// are one round of its workgroups and few rows leave each MFMA workgroup alone
+// with a long row: up to 256 rows and six tokens, Q4_K of more than 40 chunks (256
+// x 11008 18.1 / 20.0, x 14336 19.4 / 23.4; 384 rows 30 / 23; 7 tokens 25 / 23;
+// 40 chunks 17.5 / 17.6) and Q8_0 of 17 to 32 (256 x 5120 9.7 / 10.4, x 7168 10.6
+// / 12.7, x 8192 11.1 / 13.0; 16 chunks 10.7 / 8.2, 40: 17.7 / 15.3; 384 rows 14.4 /
+// 12.8).  Q4_0 is level at 56 chunks (19.5 / 19.7).
+inline bool mfd_sizes(int fmt, int rows, int cols, int T) {
+  if (fmt != NX_FMT_Q4_K && fmt != NX_FMT_Q4_0 && fmt != NX_FMT_Q8_0) return false;
+  if (T <= 4 || cols % MD_K != 0) return false;
+  const int n = cols / MD_K;
+  if (T <= 6 && rows <= 256 && ((fmt == NX_FMT_Q4_K && n > 40) || (fmt == NX_FMT_Q8_0 && n > 16 && n <= 32)))
+    return false;
+  return true;
+}
+
+// A workgroup's shape: r row tiles of 16 per wave, kw chunk groups of 8 / kw
+// waves and as many token tiles.
+struct MfdShape {
+  int r, kw;
+  int rows() const { return 16 * r * (MD_WAVES / kw); }
+  int tokens() const { return 16 * (MD_WAVES / kw); }
+};
+
+// One workgroup fits a CU (its stage fills the LDS), so a shape costs its
+// rounds of the CUs times its steps of kw chunks.  Step times (us, one
+// MI355X, all rows and tokens of a shape in use, the formats within 10%):
+// a step costs its 8 waves about 4 us of conversion, staging and waits, and
+// little more for more rows or token tiles, so the larger shapes win where
+// they fill the CUs.  4096 x 4096 Q4_K, 1 x 8 / 2 x 8 / 4 x 8 / 2 x 4 / 1 x 2 /
+// 2 x 2: 16 tokens 11.1 / 12.0 / 16.7 / 23.8 / 41.8 / 53.1 us; 64 tokens 40.3
+// / 24.5 / 18.2 / 24.4 / 41.8 / 53.4; 509 tokens 330 / 187 / 135 / 98 / 91 /
+// 62.
+inline MfdShape mfd_shape(int rows, int nchunk, int T, int num_cu) {
+  static const struct {
+    MfdShape s;
+    double step_us;
+  } shapes[] = {{{1, 8}, 4.0}, {{2, 8}, 4.5}, {{4, 8}, 6.8}, {{1, 4}, 4.4},
+                {{2, 4}, 5.2}, {{1, 2}, 4.8}, {{2, 2}, 6.2}};
+  MfdShape s{1, 8};
+  double best = 0.0;
+  for (const auto &t : shapes) {
+    const long wgs = (long)((rows + t.s.rows() - 1) / t.s.rows()) * ((T + t.s.tokens() - 1) / t.s.tokens());
+    const double us = t.step_us * (double)((wgs + num_cu - 1) / num_cu) *
+                      (double)((nchunk + t.s.kw - 1) / t.s.kw);
+    if (best == 0.0 || us < best) best = us, s = t.s;
+  }
+  return s;
 }
 
 }  // namespace nx

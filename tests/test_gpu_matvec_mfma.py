@@ -86,3 +86,17 @@ def test_unaligned_input(ctx):
     assert_close(out[:480].reshape(6, 80), w, x)
     assert out[480] == 7.0
     m.close()
+
+
+@pytest.mark.parametrize("fmt,rows,cols", [(nx.Q4_K, 256, 10496), (nx.Q4_K, 17, 14336),
+                                           (nx.Q8_0, 256, 4352), (nx.Q8_0, 48, 8192)])
+def test_few_long_rows_stay_on_the_gemv(ctx, fmt, rows, cols):
+    """Up to six tokens of at most 256 long rows: the GEMV, which gives each
+    token the bits of a call of its own."""
+    m, w = matrix(ctx, fmt, rows, cols, seed=rows + cols)
+    x = np.random.default_rng(9).standard_normal((6, cols)).astype(np.float32)
+    alone = np.concatenate([m.matvec(x[t:t + 1]) for t in range(6)])
+    for T in (5, 6):
+        assert_same_bits(m.matvec(x[:T]), alone[:T])
+    assert_close(alone, w, x)
+    m.close()

@@ -1,5 +1,6 @@
-"""What a MoE call's sizes decide (nexus_amd/csrc/nx_plan.hpp): the path AUTO
-takes and the split-activation path's workspace.  CPU only: the header is plain
+"""What a call's sizes decide (nexus_amd/csrc/nx_plan.hpp): the path AUTO takes,
+the split-activation path's workspace and runs, and the dense matvec's kernel.
+CPU only: the header is plain
 C++ and is compiled on its own with the host compiler.
 """
 import os
@@ -190,4 +191,24 @@ def test_auto_in_the_scratch_array(tmp_path):
   }
   if (auto_path(s, 101, 8, true, limit) != NX_PATH_MFMA_BF16) ++bad;
   if (auto_path(s, 101, 8, true, SIZE_MAX) != NX_PATH_MFMA_SPLIT) ++bad;
+""")
+
+
+def test_dense_kernel(tmp_path):
+    """The dense matvec runs on the matrix cores from five tokens of whole
+    256-column chunks, but for up to six tokens of at most 256 long rows."""
+    run(tmp_path, r"""
+  for (int fmt : {NX_FMT_F32, NX_FMT_F16, NX_FMT_BF16, NX_FMT_Q2_K, NX_FMT_Q4_0, NX_FMT_Q8_0, NX_FMT_Q4_K})
+    for (int rows : {1, 16, 255, 256, 257, 4096})
+      for (int cols = 32; cols <= 14336; cols += 32)
+        for (int T : {1, 4, 5, 6, 7, 16, 512}) {
+          const bool fits = fmt == NX_FMT_Q4_0 || fmt == NX_FMT_Q8_0 || fmt == NX_FMT_Q4_K;
+          const bool small = rows <= 256 && T <= 6;
+          const bool gemv = small && ((fmt == NX_FMT_Q4_K && cols > 10240) ||
+                                      (fmt == NX_FMT_Q8_0 && cols > 4096 && cols <= 8192));
+          if (mfd_sizes(fmt, rows, cols, T) != (fits && T >= 5 && cols % 256 == 0 && !gemv)) {
+            std::printf("fmt %d, %d x %d, T %d\n", fmt, rows, cols, T);
+            ++bad;
+          }
+        }
 """)
