@@ -20,8 +20,8 @@
 //     accumulates in f32.
 //   - Q4_K (src/quant/mod.rs:820-849): w = d sc (q - 8) + (8 d sc - dmin m),
 //     so a chunk's 8 sub-blocks accumulate together, the sub-block sums X_s
-//     enter one K = 16 MFMA against 8 sc_s and one against m_s, and d and dmin
-//     apply once per chunk.  Q4_0 and Q8_0 (src/quant/mod.rs:689-745): one
+//     enter one K = 16 MFMA against 8 sc_s and one against m_s, and d and
+//     dmin apply once per chunk.  Q4_0 and Q8_0 (src/quant/mod.rs:689-745): one
 //     MFMA pair per 32-weight block, whose f16 scale applies to its result.
 //
 // Work: a workgroup of 8 waves, KW chunk groups of RW = 8 / KW waves, owns 16 R
@@ -246,12 +246,13 @@ __global__ __launch_bounds__(64 * MD_WAVES, 2) void k_mfd(const MfdArgs a) {
         for (int n = 0; n < NT; ++n) {
           const f16x4 xm = *reinterpret_cast<const f16x4 *>(&st[n].xm[lane]);
           const f32x4 sx = *reinterpret_cast<const f32x4 *>(&st[n].sx[4 * g]);
-          y[r][n] = __builtin_amdgcn_mfma_f32_16x16x16f16(xm, f16x4{b0, b0, b1, b1}, y[r][n], 0, 0, 0);
-          const f32x4 ym = __builtin_amdgcn_mfma_f32_16x16x16f16(xm, f16x4{m0, m0, m1, m1},
-                                                                 f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+          // (never onto y: nx_mfv.hip)
+          const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+          const f32x4 yx = __builtin_amdgcn_mfma_f32_16x16x16f16(xm, f16x4{b0, b0, b1, b1}, zero, 0, 0, 0);
+          const f32x4 ym = __builtin_amdgcn_mfma_f32_16x16x16f16(xm, f16x4{m0, m0, m1, m1}, zero, 0, 0, 0);
 #pragma unroll
           for (int k = 0; k < 4; ++k)
-            acc[r][n][k] = fmaf(sx[k], fmaf(dd, y[r][n][k], -dm * ym[k]), acc[r][n][k]);
+            acc[r][n][k] = fmaf(sx[k], fmaf(dd, y[r][n][k], fmaf(dd, yx[k], -dm * ym[k])), acc[r][n][k]);
         }
       }
     } else {

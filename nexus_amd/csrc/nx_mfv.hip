@@ -303,22 +303,32 @@ __global__ __launch_bounds__(64 * MV_KW, 2) void k_mfv(const MfvArgs a) {
           const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(w.m.x & 0xFFFF));
           const float dmin = (float)__builtin_bit_cast(_Float16, (uint16_t)(w.m.x >> 16));
           const float dd = d * 16384.0f, dm = dmin * 64.0f;  // X enters 2^-6
-          f32x4 ym;
+          const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+          f32x4 rest;  // what the offsets and mins add
           if constexpr (Q2K) {
-            ym = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+            const f32x4 ym = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                 __builtin_bit_cast(f16x8, xm), f16x8{mn[0], mn[0], mn[1], mn[1], mn[NV - 2], mn[NV - 2], mn[NV - 1], mn[NV - 1]},
-                f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                zero, 0, 0, 0);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) rest[k] = -dm * ym[k];
           } else {
-            // 8 sc X at the codes' 2^-14 (X enters 2^-6): sc 2^-5; and m
+            // 8 sc X at the codes' 2^-14 (X enters 2^-6): sc 2^-5; and m.  On
+            // accumulators of their own: the result of an MFMA of one shape, taken
+            // as another shape's accumulator, is read before it is complete unless
+            // enough instructions lie between, and the compiler (ROCm 7.2) puts no
+            // wait there.  16x16x32 and 16x16x16 back to back on one accumulator
+            // lose the first in two of the four registers.
             const f16x4 xa = __builtin_bit_cast(f16x4, uint2{xm.x, xm.y});
             const _Float16 k15 = (_Float16)0x1p-15f;
             const _Float16 b0 = s1[0][0] * k15, b1 = s1[NV - 1][0] * k15;
-            y = __builtin_amdgcn_mfma_f32_16x16x16f16(xa, f16x4{b0, b0, b1, b1}, y, 0, 0, 0);
-            ym = __builtin_amdgcn_mfma_f32_16x16x16f16(xa, f16x4{mn[0], mn[0], mn[NV - 1], mn[NV - 1]},
-                                                       f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            const f32x4 yx = __builtin_amdgcn_mfma_f32_16x16x16f16(xa, f16x4{b0, b0, b1, b1}, zero, 0, 0, 0);
+            const f32x4 ym = __builtin_amdgcn_mfma_f32_16x16x16f16(
+                xa, f16x4{mn[0], mn[0], mn[NV - 1], mn[NV - 1]}, zero, 0, 0, 0);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) rest[k] = fmaf(dd, yx[k], -dm * ym[k]);
           }
 #pragma unroll
-          for (int k = 0; k < 4; ++k) res[k] = sx[k] * fmaf(dd, y[k], -dm * ym[k]);
+          for (int k = 0; k < 4; ++k) res[k] = sx[k] * fmaf(dd, y[k], rest[k]);
         }
         __builtin_amdgcn_sched_barrier(0);
         issue(ring[(i + D) % MV_STEPS], i + D < MV_STEPS ? rt : rt + RT, (i + D) % MV_STEPS);
