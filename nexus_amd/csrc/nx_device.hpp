@@ -38,6 +38,16 @@ __device__ __forceinline__ float h2f(uint32_t bits16) {
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
+// Between LDS stores of a wave's lanes and other lanes' loads of them.  A wave's
+// LDS operations complete in order, so nothing is waited for; the fences keep
+// the compiler from reordering accesses that it can prove apart within one lane
+// (the wave barrier alone orders no memory).
+__device__ __forceinline__ void wave_handoff() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+}
+
 // Raw buffer resources: 32-bit byte offsets, and any load at or beyond
 // `bytes` returns zeros instead of touching memory, so out-of-range rows and
 // segments need no branches.

@@ -164,7 +164,7 @@ __global__ __launch_bounds__(64 * MD_WAVES, 2) void k_mfd(const MfdArgs a) {
     if constexpr (RW > 1)
       __syncthreads();
     else
-      __builtin_amdgcn_wave_barrier();
+      wave_handoff();
   };
 
   f32x4 acc[R][NT];

@@ -130,9 +130,8 @@ __global__ __launch_bounds__(256) void k_rms_runs(const float *__restrict__ x,
       my[pad(i)] = v[j];
     }
   }
-  // the runs below read other lanes' staged float4s: keep every staging
-  // store of the wave ahead of them (a wave's LDS accesses complete in order)
-  __builtin_amdgcn_wave_barrier();
+  // the runs below read other lanes' staged float4s
+  wave_handoff();
   float ss = 0.f;
   {
     float4 q[S4];
