@@ -101,7 +101,7 @@ __device__ __forceinline__ float split16(const f32x4 (&v)[4], int j16, Put put, 
   mx = fmaxf(mx, dpp_f<0x121>(mx));
   // max|x| < 2^E; an infinity or NaN ends as NaN through x' - hi or hi
   int E = mx < INFINITY ? __builtin_amdgcn_frexp_expf(mx) : 0;
-  E = max(E, -100);
+  E = max(E, -112);  // 2^126 and 2^-126 at most: smaller maxima keep their bits down to 2^-126
   const float up = __builtin_amdgcn_ldexpf(1.0f, 14 - E);
   const int kd = (j16 >> 1) & 3, s0 = j16 >> 3;
 #pragma unroll

@@ -100,3 +100,18 @@ def test_few_long_rows_stay_on_the_gemv(ctx, fmt, rows, cols):
         assert_same_bits(m.matvec(x[:T]), alone[:T])
     assert_close(alone, w, x)
     m.close()
+
+
+@pytest.mark.parametrize("fmt", [nx.Q4_K, nx.Q4_0, nx.Q8_0])
+def test_smallest_normal_values(ctx, fmt):
+    """Tokens of the smallest normal numbers keep the precision of others: their
+    scaled maximum is at least 1, whose two halves reach 2^-25, so the error of
+    a value is some 2^-24 of the maximum and a sum's relative error below 2^-20."""
+    m, w = matrix(ctx, fmt, 64, 512, seed=fmt + 5)
+    x = np.random.default_rng(7).standard_normal((9, 512)).astype(np.float32)
+    x *= np.logspace(-37, -34, 9, dtype=np.float32)[:, None]
+    got = m.matvec(x).astype(np.float64)
+    ref = x.astype(np.float64) @ w.T
+    err = np.linalg.norm(got - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert np.all(err < 2.0 ** -20), err
+    m.close()
