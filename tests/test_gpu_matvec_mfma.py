@@ -1,9 +1,11 @@
 """Dense matvec of five and more tokens on the matrix cores (nx_mfd.hip).
 
 Against the oracle's dequantization of the same payload in 64 bits.  The
-sizes cover each instance (1, 2 and 4 row tiles of 16, one or two token
-tiles), ragged last row and token tiles, fewer chunks of 256 columns than a
-workgroup has waves, and rows of several panels.
+sizes cover ragged last row and token tiles, fewer chunks of 256 columns than a
+workgroup has waves, rows of several panels, and in INSTANCES each instance on
+256 CUs (1, 2 or 4 row tiles of 16 per wave; 8, 4 or 2 chunk groups with 1, 2 or
+4 token tiles) over several steps of which the last is ragged; test_plan.py
+checks that those sizes choose them.
 
 Bound per output: the operands carry 22 bits, and a product is rounded at
 most some 2^5 times on its way (8 MFMAs, the chunks and the 8 waves' sums), so
@@ -42,6 +44,26 @@ def assert_close(got, w, x):
     bound = 2.0 ** -18 * np.linalg.norm(x, axis=1)[:, None] * np.linalg.norm(w, axis=1)[None, :]
     err = np.abs(got - x @ w.T)
     assert np.all(err <= bound), np.nanmax(err / np.maximum(bound, 1e-300), axis=1)
+
+
+# row tiles per wave, chunk groups, and a size that chooses them
+INSTANCES = [(1, 8, 37, 2304, 5), (2, 8, 325, 2304, 200), (4, 8, 500, 3328, 260), (1, 4, 325, 2304, 400),
+             (2, 4, 1000, 2304, 260), (1, 2, 1335, 1280, 400), (2, 2, 8197, 1280, 65)]
+
+
+@pytest.mark.parametrize("fmt", [nx.Q4_K, nx.Q4_0, nx.Q8_0])
+@pytest.mark.parametrize("case", INSTANCES, ids=lambda c: "%dx%d-%d-%d-%d" % c)
+def test_instances(ctx, fmt, case):
+    print(f"matvec instance fmt={nx.FORMAT_NAMES[fmt]} {case}", flush=True)
+    rows, cols, T = case[2:]
+    m, w = matrix(ctx, fmt, rows, cols, seed=rows + cols + T + fmt)
+    x = np.random.default_rng(T).standard_normal((T, cols)).astype(np.float32)
+    got = m.matvec(x)
+    assert_close(got, w, x)
+    # and as close to 64 bits as the kernel's error elsewhere (2.1e-7), per token
+    ref = x.astype(np.float64) @ w.T
+    assert np.all(np.linalg.norm(got - ref, axis=1) < 2.0 ** -20 * np.linalg.norm(ref, axis=1))
+    m.close()
 
 
 @pytest.mark.parametrize("fmt", [nx.Q4_K, nx.Q4_0, nx.Q8_0])

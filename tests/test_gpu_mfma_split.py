@@ -1,7 +1,7 @@
 """Few-token MoE layer on MFMA with split-fp16 activations (NX_PATH_MFMA_SPLIT).
 
-The Q4_K codes go into fp16 MFMA operands untouched (no dequantization) and
-each 32-weight sub-block's scale and offset are applied to the products;
+The Q4_K codes go into fp16 MFMA operands times their sub-block's scale (exact,
+no dequantization), and the block's scales and offsets are applied to the sums;
 activations are split per pair and 256-element chunk into two fp16 halves
 after a power-of-two scaling.  Bar: the GEMV path's, relative L2 1e-4
 against the oracle's dispatch (src/engine/mod.rs:969-1024) over the same
@@ -106,8 +106,8 @@ def test_split_mixtral_shape(ctx):
 def test_split_parity_block_formats(ctx, fmt, E, H, F, k, T, Fs, score):
     """Q4_0 experts (w = d (q - 8) per 32-weight block, src/quant/mod.rs:
     723-745) and Q8_0 experts (w = d q, q a signed byte, :689-703) on the
-    split path: one MFMA per block with the codes made unsigned, the block
-    sums of the staged activations taking off the offset (8, 128)."""
+    split path: an MFMA pair per block on the signed codes as fp16 values, the
+    block's scale applied to its result."""
     print(f"mfma split fmt={fmt} E={E} H={H} F={F} k={k} T={T} Fs={Fs} score={score}", flush=True)
     L = Layer(fmt, E, H, F, k, T, seed=E * 3 + H + F + T + fmt, shared_F=Fs, score_mode=score)
     ex = L.upload(nx, ctx)
@@ -200,9 +200,9 @@ def test_split_rejects(ctx):
     (8, 512, 1024, 2, 16, nx.PATH_MFMA_SPLIT), (64, 256, 256, 8, 8, nx.PATH_MFMA_SPLIT),
     (8, 256, 256, 2, 64, nx.PATH_MFMA_BF16), (8, 256, 256, 2, 256, nx.PATH_MFMA_BF16)])
 def test_auto_path_choice(ctx, E, H, F, k, T, want):
-    """AUTO gives the bits of the path it chooses for Q4_K: the GEMV up to ~2
-    tokens per expert, the split-activation MFMA path up to ~12, the grouped
-    GEMM beyond."""
+    """AUTO gives the bits of the path it chooses for Q4_K in small layers: the
+    GEMV below 3 tokens per expert (1.2 from 64 pairs), the split-activation MFMA
+    path up to 12, the grouped GEMM beyond.  Large layers: test_gpu_auto_paths.py."""
     L = Layer(Q4_K, E, H, F, k, T, seed=E + T)
     ex = L.upload(nx, ctx)
     auto = ex.forward(L.x, L.logits, k, 0, nx.PATH_AUTO)
@@ -235,15 +235,15 @@ def test_auto_path_choice(ctx, E, H, F, k, T, want):
     (Q4_K, 4, 256, 256, 2, 48, 256, nx.PATH_MFMA_BF16),   # ... 24 tokens per routed expert
     (Q4_K, 16, 512, 512, 4, 8, 1024, nx.PATH_MFMA_BF16)])  # a wider shared expert, 8 tokens
 def test_auto_path_choice_other(ctx, fmt, E, H, F, k, T, shared, want):
-    """AUTO for formats other than Q4_K and for layers with a shared expert:
-    the grouped GEMM from ~3 tokens per routed expert, or from 6 tokens with
-    a shared expert, the GEMV below; Q4_0 and Q8_0 without a shared expert,
-    in whole 256-weight chunks, follow Q4_K's rule (split path from ~3 tokens per
-    expert up to 12); Q2_K takes the split path from ~1.8 tokens per expert
-    (or 4 tokens with a shared expert as wide as the routed ones), the GEMV
-    below; Q4_K with a shared expert as wide as the routed ones
-    takes the split-activation path from 4 tokens up to 8 tokens per routed
-    expert (the bits of the chosen path)."""
+    """AUTO for formats other than Q4_K and for layers with a shared expert, all
+    of them small (large layers: test_gpu_auto_paths.py): the grouped GEMM from ~3
+    tokens per routed expert, or from 6 tokens with a shared expert, the GEMV
+    below; Q4_0 and Q8_0 without a shared expert, in whole 256-weight chunks,
+    follow Q4_K's rule (split path from ~3 tokens per expert up to 12); Q2_K takes
+    the split path from ~1.8 tokens per expert (or 4 tokens with a shared expert
+    as wide as the routed ones), the GEMV below; Q4_K with a shared expert as wide
+    as the routed ones takes the split-activation path from 4 tokens up to 8
+    tokens per routed expert (the bits of the chosen path)."""
     L = Layer(fmt, E, H, F, k, T, seed=E + T + fmt, shared_F=shared)
     ex = L.upload(nx, ctx)
     auto = ex.forward(L.x, L.logits, k, 0, nx.PATH_AUTO)

@@ -212,3 +212,25 @@ def test_dense_kernel(tmp_path):
           }
         }
 """)
+
+
+def test_dense_instances(tmp_path):
+    """The sizes of the dense matvec's instance test choose each of the seven
+    instances on 256 CUs, over several steps with a ragged last one."""
+    from test_gpu_matvec_mfma import INSTANCES
+
+    assert len({c[:2] for c in INSTANCES}) == 7
+    rows = ",".join("{%d, %d, %d, %d, %d}" % c for c in INSTANCES)
+    run(tmp_path, r"""
+  const struct { int r, kw, rows, cols, T; } cases[] = {""" + rows + r"""};
+  for (const auto &c : cases) {
+    const int n = c.cols / MD_K;
+    const MfdShape s = mfd_shape(c.rows, n, c.T, 256);
+    for (int fmt : {NX_FMT_Q4_K, NX_FMT_Q4_0, NX_FMT_Q8_0})
+      if (!mfd_sizes(fmt, c.rows, c.cols, c.T)) ++bad;
+    if (s.r != c.r || s.kw != c.kw || n <= s.kw || n % s.kw == 0 || c.rows % s.rows() == 0 || c.T % s.tokens() == 0) {
+      std::printf("%d x %d, %d tokens: %d x %d\n", c.rows, c.cols, c.T, s.r, s.kw);
+      ++bad;
+    }
+  }
+""")
