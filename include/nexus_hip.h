@@ -96,7 +96,7 @@ extern "C" {
 #define NX_PATH_MFMA_F16 2  /* grouped GEMM on fp16 MFMA, fp32 accumulate; activations and
                                SwiGLU outputs must stay within fp16's range (|v| < 65504) */
 #define NX_PATH_MFMA_BF16 3 /* same on bf16 MFMA */
-#define NX_PATH_MFMA_SPLIT 4 /* few tokens per expert (decode batches), Q4_K, Q2_K, or Q4_0 and
+#define NX_PATH_MFMA_SPLIT 4 /* few tokens per expert (up to ~13), Q4_K, Q2_K, or Q4_0 and
                                 Q8_0 whose hidden and ff dims are multiples of 256: fp16 MFMA
                                 on the raw codes with activations split into two fp16 halves,
                                 block and sub-block scales applied to the products; no
@@ -227,9 +227,11 @@ int nx_matrix_destroy(nx_matrix *m);
 /* y[t * rows + r] = sum_c W[r][c] x[t * cols + c] for T = num_tokens, fp32
  * in and out: InferenceEngine::matvec (src/engine/mod.rs:775-801) on each
  * token row, with the dot product in parallel order (fp32 accumulate) over
- * the quantized codes.  Five and more tokens of Q4_K, Q4_0 or Q8_0 rows of
- * whole 256-weight chunks run on the matrix cores, within the same error, so a
- * token's last bits can differ between the two.  x_len != T*cols gives NX_ERR_SHAPE
+ * the quantized codes.  Up to four tokens get the bits of calls of their own.
+ * Most calls of five and more tokens on Q4_K, Q4_0 or Q8_0 rows of whole
+ * 256-weight chunks run on the matrix cores, within the same error, and there a
+ * token's last bits depend on the number of tokens and rows (the order of the
+ * sums does).  x_len != T*cols gives NX_ERR_SHAPE
  * "Matvec input shape mismatch: got <x_len>, expected <T*cols>". */
 int nx_matvec(nx_ctx *ctx, const nx_matrix *m, const float *x, size_t x_len, int num_tokens,
               float *y);

@@ -36,10 +36,13 @@
 //
 // Bound by instruction issue: a wave's share of the conversion (about 450
 // instructions per token tile and chunk) and of the operands, with two waves
-// per SIMD (registers, LDS) to cover each other's waits; the matrix cores are
-// busy a quarter of the time.  Measured against the GEMV (us): 4096 x 4096
-// Q4_K, 5 tokens 13.3 -> 10.0, 64 tokens 112 -> 17.4, 509 tokens 870 -> 59;
-// 32000 x 4096 Q8_0, 13 tokens 160 -> 44 (3.2 TB/s of weights).  Error against
+// per SIMD (registers, LDS) to cover each other's waits.  Counters, 4096 x 4096
+// Q4_K, 509 tokens: 60% of the issue slots taken, the matrix cores busy 25% of
+// the time, waves waiting 27% of theirs for memory or a barrier and 36% for
+// issue; 32000 x 4096 Q8_0, 13 tokens: 38%, 7%, 32% and 43%.  Measured against
+// the GEMV (us): 4096 x 4096 Q4_K, 5 tokens 12.8 -> 9.2, 64 tokens 112 -> 17.0,
+// 509 tokens 874 -> 54-58; 32000 x 4096 Q8_0, 13 tokens 159 -> 44.5 (3.2 TB/s of
+// weights).  Error against
 // 64 bits 2.1e-7 (Q4_K) and 1.1e-7 (Q4_0, Q8_0), the GEMV's 3.0e-7 and 2.7e-7.
 #include "nx_internal.hpp"
 #include "nx_split_dev.hpp"

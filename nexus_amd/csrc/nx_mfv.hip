@@ -36,16 +36,16 @@
 // weight rows past them, the codes of the next MV_D steps in flight.  The waves
 // of a workgroup take the chunks of one K slice (at most 8) side by side, so
 // the 128-byte lines that two chunks' codes and eight chunks' scales share are
-// read at about the same time, and add their results through LDS every four
-// steps.  Slices write partial sums, which the SwiGLU kernel (gate/up) and the
+// read at about the same time, and add their results through LDS every pass
+// of four steps.  Slices write partial sums, which the SwiGLU kernel (gate/up) and the
 // weighted combine (down) add in slice order.
 //
 // Bound by the weight stream, then by instruction issue: Mixtral Q4_K, 32
 // tokens, gate/up (529 MB) 127 us, of which the loads alone take 123 and the
 // arithmetic alone 99.  Against workgroups of 256 rows that staged their
 // activations in LDS and walked a slice of 4 chunks (us, layer): Mixtral 32
-// tokens 247 -> 211, DeepSeek 27 tokens 1008 -> 806, Qwen3 61 tokens 118.6 ->
-// 108; error against 64 bits 9.3e-7 -> 3.9e-7 (Q4_K), 7.8e-5 -> 2.1e-7 (Q4_0,
+// tokens 246 -> 212, DeepSeek 27 tokens 1049 -> 836, Qwen3 61 tokens 118.5 ->
+// 108.9; error against 64 bits 9.3e-7 -> 3.8e-7 (Q4_K), 7.8e-5 -> 2.1e-7 (Q4_0,
 // whose codes were fp16 subnormals).  A wave per 64 rows that walked the chunks
 // itself read each line's halves a chunk apart, too late for the L2: 370 us.
 #include "nx_internal.hpp"
