@@ -111,7 +111,7 @@ inline int auto_path(const MoeShape &s, int T, int k, bool aligned, size_t scrat
   const double act = std::max(1.0, s.E * (1.0 - std::pow(1.0 - kk, (double)T)));
   const double tpe = (double)T * k / act;
   // The split path streams the active experts' weights at 4.3 TB/s behind
-  // about 35 us of launches, so it wins over wider ranges where an expert is
+  // about 30 us of launches, so it wins over wider ranges where an expert is
   // large: `large` from 7 M weights a matrix (measured at 4096 x 1792 and up).
   // In the fixed scratch array of nx_moe_forward_noalloc a batch that its
   // workspace would not fit keeps the narrower ranges, whose other paths
@@ -125,11 +125,10 @@ inline int auto_path(const MoeShape &s, int T, int k, bool aligned, size_t scrat
   const bool q8 = s.fmt == NX_FMT_Q8_0;
   if (s.fmt == NX_FMT_Q2_K) {
     // The GEMV or the split-activation path (Q2_K has no grouped GEMM).
-    // Measured (ms, GEMV / split): Mixtral 2 tokens 0.101 / 0.122, 4:
-    // 0.173 / 0.188, 8: 0.243 / 0.193, 32: 0.939 / 0.238, 128: 2.82 /
-    // 0.534; Qwen3 4 tokens 0.048 / 0.048, 8: 0.093 / 0.065, 512: 1.84 /
-    // 0.265; DeepSeek with its shared expert 2 tokens 0.119 / 0.137, 4:
-    // 0.307 / 0.218, 64: 44.1 / 1.52.
+    // Measured (us, GEMV / split): Mixtral 2 tokens 93 / 84, 4: 174 / 112, 8:
+    // 276 / 153, 32: 797 / 170, 128: 2840 / 364; Qwen3 4 tokens 46 / 40, 8: 77 /
+    // 52, 128: 588 / 97; DeepSeek with its shared expert 2 tokens 121 / 104, 4:
+    // 305 / 175.  (The limits are those of a slower split kernel.)
     if (!split_fmt) return NX_PATH_GEMV;
     if (shared) return (s.Fs == s.F && T >= 4) ? NX_PATH_MFMA_SPLIT : NX_PATH_GEMV;
     return (tpe >= 1.8 || ((long)T * k >= 64 && tpe >= 1.2)) ? NX_PATH_MFMA_SPLIT : NX_PATH_GEMV;
@@ -137,12 +136,12 @@ inline int auto_path(const MoeShape &s, int T, int k, bool aligned, size_t scrat
   if (split_fmt && shared && s.Fs == s.F && (large || s.fmt == NX_FMT_Q4_K)) {
     // A shared expert sees every token: the GEMV walks it a token pair at
     // a time, the split-activation path 16 tokens at a time.  Measured
-    // (DeepSeek shapes, us, GEMV / split / grouped GEMM): Q4_K 2 tokens 105
-    // / 128 / 233, 4: 265 / 196 / 282, 27: 9257 / 836 / 1251, 128: - / 1546 /
-    // 1989, 256 (8 per routed expert): - / 1836 / 2090, 400 (12.5): - / 2105
-    // / 2123; Q4_0 4: 232 / 198 / 281, 27: - / 950 / 1226, 128: - / 1665 /
-    // 1960; Q8_0 8: 840 / 542 / 643, 27: - / 1357
-    // / 1524, 300 (9.4): - / 2924 / 2730.
+    // (DeepSeek shapes, us, GEMV / split / grouped GEMM): Q4_K 2 tokens 107 /
+    // 117 / 238, 4: 263 / 183 / 283, 8: 874 / 331 / 580, 27: - / 867 / 1262,
+    // 128: - / 1562 / 2018, 256 (8 per routed expert): - / 1794 / 2122, 384
+    // (12): - / 1952 / 2151; Q4_0 2: 98 / 123 / 235, 4: 237 / 204 / 364, 27: - /
+    // 842 / 1241, 384: - / 1937 / 2104; Q8_0 4: 315 / 323 / 450, 8: 847 / 557 /
+    // 676, 128: - / 2425 / 2554, 256: - / 2772 / 2702.
     if (tpe >= (large && !q8 ? 12.0 : 8.0)) return NX_PATH_MFMA_BF16;
     return T >= (q8 ? 6 : 4) ? NX_PATH_MFMA_SPLIT : NX_PATH_GEMV;
   }
@@ -150,29 +149,27 @@ inline int auto_path(const MoeShape &s, int T, int k, bool aligned, size_t scrat
     // The GEMV re-reads an expert's weights per pair of its tokens, the
     // split-activation path reads them once per 16 tokens, and the grouped
     // GEMM once, at bf16 operands.  Measured (us, GEMV / split / grouped
-    // GEMM) by tokens per expert: Mixtral Q4_0 1.1: 80 / 96 / 176, 1.5: 154 /
-    // 130 / 240, 2.0: 249 / 155 / 244; Q4_K 1.3: 128 / 107 / 201, 2.2: 454 /
-    // 156 / 254, 8: 906 / 215 / 301, 12: - / 241 / 304, 16: - / 320 / 305;
-    // Q8_0 2.0: 320 / 239 / 295, 8: - / 338 / 363, 16: - / 540 / 365; Qwen3
-    // Q4_K 1.1: 45 / 50 / 68, 1.3: 107 / 64 / 93, 8: - / 132 / 151, 12.5: -
-    // / 137 / 153, 16: - / 155 / 156.  Smaller layers (GEMV / split): 8
-    // experts of 4096 x 1792 Q4_K 1.3: 38 / 37, 1.6: 57 / 43, Q8_0 1.6: 48 /
-    // 54, 2.2: 59 / 54; 1024 x 2048 Q4_K 1.3: 31 / 35, 1.6: 42 / 35; 512 x
-    // 1024 Q4_K 1.6: 25 / 34, 2.2: 35 / 36, 3.1: 46 / 37; 64 experts of 1024
-    // x 768, top 8, 1.1: 35 / 35, 1.3: 53 / 36.
-    // The GEMV's time hangs on how the tokens pair up, so the lower limits are
-    // from means over eight routings (GEMV / split): large layers Q4_K 1.3:
-    // Mixtral 136 / 113, 16 experts of 4096 x 2304 61 / 57; Q4_0 1.3: 102 / 117
-    // and 51 / 61, 1.46: 138 / 132 and 69 / 65; Q8_0 2.0: 286 / 255 and 136 /
-    // 110.  Of 7 M weights: 4 experts of 2048 x 3584 Q4_K 6 pairs 34 / 36, 8
-    // pairs 40 / 37, Q8_0 10 pairs 42 / 43; 8 of 4096 x 1792 Q4_K 6 pairs 37 /
-    // 40, 8 pairs 46 / 43, Q8_0 14 pairs 52 / 56, 16 pairs 61 / 57.  64 of 1024
-    // x 768 Q8_0 1.28: 38 / 42, 1.36: 49 / 45.
+    // GEMM, means over four to thirty routings: the GEMV's time hangs on how the
+    // tokens pair up) by tokens per expert.  Mixtral Q4_K 1.1: 90 / 94 / 176,
+    // 1.3: 150 / 115 / 223, 2.2: 382 / 172 / 296, 8: - / 213 / 305, 12: - / 225 /
+    // 307, 16: - / 271 / 314; Q4_0 1.3: 99 / 114 / 216, 1.46: 130 / 132 / 243,
+    // 1.64: 160 / 144 / -, 12: - / 232 / 300; Q8_0 1.5: 193 / 213 / 286, 2.0: 300
+    // / 265 / 338, 8: - / 344 / 364, 12: - / 370 / 368, 16: - / 463 / 369; Qwen3
+    // Q4_K 1.1: 51 / 44 / 68, 1.3: 124 / 61 / 93, 8: - / 123 / 152, 12.5: - / 136 /
+    // 154, 16: - / 154 / 156.  16 experts of 4096 x 2304, top 4, 1.3: Q4_K 61 /
+    // 57, Q4_0 51 / 61; 1.46: Q4_0 68 / 65; 2.0: Q8_0 129 / 111.
+    // Layers of 7 M weights, 4 experts of 2048 x 3584: Q4_K 6 pairs 34 / 36, 8
+    // pairs 40 / 37, Q8_0 10 pairs 42 / 43; 8 of 4096 x 1792: Q4_K 6 pairs 37 /
+    // 39, 8 pairs 45 / 43, Q8_0 14 pairs 52 / 56, 16 pairs 61 / 56.  Smaller ones:
+    // 8 of 1024 x 2048 Q4_K 1.5: 34 / 32, 1.6: 41 / 32, Q8_0 2.2: 33 / 37, 3.1: 40
+    // / 38; 8 of 512 x 1024 Q4_K 1.6: 30 / 30, 2.2: 36 / 31, Q8_0 3.1: 35 / 36; 64
+    // of 1024 x 768, top 8, Q4_K 1.1: 31 / 31, 1.3: 47 / 37, Q8_0 1.28: 38 / 42,
+    // 1.36: 49 / 45.
     const long pairs = (long)T * k;
     if (tpe >= (large && !q8 ? 13.0 : 12.0)) return NX_PATH_MFMA_BF16;
     // the least tokens per expert of a large layer; the smallest of them with a
     // few pairs are bound by the launches, of which the GEMV has fewer
-    const double least = q8 ? 2.0 : s.fmt == NX_FMT_Q4_0 ? 1.4 : 1.28;
+    const double least = q8 ? 2.0 : s.fmt == NX_FMT_Q4_0 ? 1.5 : 1.28;
     const bool few = weights < 9e6 && pairs < (q8 ? 16 : 8);
     if (tpe >= 3.0 || (pairs >= 64 && tpe >= 1.2) || (fits && pairs >= 40 && tpe >= (q8 ? 1.3 : 1.25)) ||
         (large && !few && tpe >= least) || (fits && !q8 && !few && weights >= 2e6 && tpe >= 1.6))

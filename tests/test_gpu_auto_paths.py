@@ -90,7 +90,7 @@ def test_unaligned_input(ctx, case):
 CHOICE = [
     (Q4_K, 8, 2048, 4608, 2, 0, 2, GEMV), (Q4_K, 8, 2048, 4608, 2, 0, 3, SPLIT),
     (Q4_K, 8, 2048, 4608, 2, 0, 51, SPLIT), (Q4_K, 8, 2048, 4608, 2, 0, 53, BF16),
-    (Q4_0, 8, 2048, 4608, 2, 0, 3, GEMV), (Q4_0, 8, 2048, 4608, 2, 0, 4, SPLIT),
+    (Q4_0, 8, 2048, 4608, 2, 0, 4, GEMV), (Q4_0, 8, 2048, 4608, 2, 0, 5, SPLIT),
     (Q4_0, 8, 2048, 4608, 2, 0, 51, SPLIT), (Q4_0, 8, 2048, 4608, 2, 0, 53, BF16),
     (Q8_0, 8, 2048, 4608, 2, 0, 6, GEMV), (Q8_0, 8, 2048, 4608, 2, 0, 7, SPLIT),
     (Q8_0, 8, 2048, 4608, 2, 0, 47, SPLIT), (Q8_0, 8, 2048, 4608, 2, 0, 49, BF16),
