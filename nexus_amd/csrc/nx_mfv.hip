@@ -102,259 +102,261 @@ __global__ __launch_bounds__(64 * MV_KW, 2) void k_mfv(const MfvArgs a) {
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // The work is a line of (tile, slice, pass of RT row tiles); each workgroup
-  // takes an equal run of it.  (Workgroups of a fixed run of rows, sized on the
+  // The work is a line of (tile, slice, pass of RT row tiles), cut into the runs
+  // of the workgroups (mfv_run).  (Workgroups of a fixed run of rows, sized on the
   // host from the expected tile count, left CUs idle wherever the routing
   // drew another: Mixtral 32 tokens 223 us, Qwen3 61 tokens 135 us.)  Passes are
-  // as short as the steps in flight allow, and few segments are not shared out
-  // across their ends (mfv_run): a run of one or two passes more than the
-  // others' is the round's tail.  Equal runs of 8-step passes took (layer, 8
+  // as short as the steps in flight allow: a run of one or two passes more than
+  // the others' is the round's tail.  Equal runs of 8-step passes took (layer, 8
   // experts, top 2) 1024 x 2048 Q8_0 256 tokens 97 us, now 75; 2048 x 1280 Q4_K
   // 128 tokens 68, now 56.
   const int ntile = a.tiles[0], npass = (a.rows >> 4) / RT;
-  const MfvRun run = mfv_run((int)blockIdx.x, (int)gridDim.x, ntile * a.nks, npass);
   int buf = 0;  // the sums' buffer of this pass: red + 0 or + ks MV_STEPS 64
-  for (long un = run.u0; un < run.u1;) {
-    const int seg = (int)(un / npass), pass0 = (int)(un - (long)seg * npass);
-    const int pass1 = (int)min((long)npass, pass0 + (run.u1 - un));
-    un += pass1 - pass0;
-    const int tile = seg / a.nks, slice = seg - tile * a.nks;
-    // tile t: expert tiles[2 + 2t] (E: the shared expert), first pair
-    // tiles[3 + 2t] within the expert
-    const int e = __builtin_amdgcn_readfirstlane(a.tiles[2 + 2 * tile]);
-    const int m0 = __builtin_amdgcn_readfirstlane(a.tiles[3 + 2 * tile]);
-    const bool routed = e < a.E;
-    const int pair0 = __builtin_amdgcn_readfirstlane(routed ? a.offsets[e] + m0 : a.T * a.k + m0);
-    const int cnt = __builtin_amdgcn_readfirstlane(
-        min(MV_M, routed ? a.offsets[e + 1] - pair0 : a.T - m0));
-    // this wave's chunk; past the row's end (the last slice) it adds zeros
-    const int c = slice * a.ks + wave;
-    const bool in_row = c < a.nchunk;
-    const int rt0 = pass0 * RT, rt1 = pass1 * RT;
+  // rounds of the segments (a tile's K slice) from `first` on
+  for (int first = 0, left = ntile * a.nks; left > 0; first += gridDim.x, left -= gridDim.x) {
+    const MfvRun run = mfv_run((int)blockIdx.x, (int)gridDim.x, left, npass);
+    for (int un = run.u0; un < run.u1;) {
+      const int s = un / npass, pass0 = un - s * npass;
+      const int pass1 = min(npass, pass0 + (run.u1 - un));
+      un += pass1 - pass0;
+      const int seg = first + run.seg0 + s, tile = seg / a.nks, slice = seg - tile * a.nks;
+      // tile t: expert tiles[2 + 2t] (E: the shared expert), first pair
+      // tiles[3 + 2t] within the expert
+      const int e = __builtin_amdgcn_readfirstlane(a.tiles[2 + 2 * tile]);
+      const int m0 = __builtin_amdgcn_readfirstlane(a.tiles[3 + 2 * tile]);
+      const bool routed = e < a.E;
+      const int pair0 = __builtin_amdgcn_readfirstlane(routed ? a.offsets[e] + m0 : a.T * a.k + m0);
+      const int cnt = __builtin_amdgcn_readfirstlane(
+          min(MV_M, routed ? a.offsets[e + 1] - pair0 : a.T - m0));
+      // this wave's chunk; past the row's end (the last slice) it adds zeros
+      const int c = slice * a.ks + wave;
+      const bool in_row = c < a.nchunk;
+      const int rt0 = pass0 * RT, rt1 = pass1 * RT;
 
-    const int l16 = lane & 15, g = lane >> 4;
-    __amdgpu_buffer_rsrc_t rq[GATEUP ? 2 : 1], rm[GATEUP ? 2 : 1];
-    {
-      const uint32_t nq = (uint32_t)a.rows * a.row_qs, nm = (uint32_t)a.rows * a.row_meta;
-      rq[0] = make_rsrc(routed ? a.qs0 + (size_t)e * a.qs_stride : a.sqs0, nq);
-      rm[0] = make_rsrc(routed ? a.meta0 + (size_t)e * a.meta_stride : a.smeta0, nm);
-      if constexpr (GATEUP) {
-        rq[1] = make_rsrc(routed ? a.qs1 + (size_t)e * a.qs_stride : a.sqs1, nq);
-        rm[1] = make_rsrc(routed ? a.meta1 + (size_t)e * a.meta_stride : a.smeta1, nm);
+      const int l16 = lane & 15, g = lane >> 4;
+      __amdgpu_buffer_rsrc_t rq[GATEUP ? 2 : 1], rm[GATEUP ? 2 : 1];
+      {
+        const uint32_t nq = (uint32_t)a.rows * a.row_qs, nm = (uint32_t)a.rows * a.row_meta;
+        rq[0] = make_rsrc(routed ? a.qs0 + (size_t)e * a.qs_stride : a.sqs0, nq);
+        rm[0] = make_rsrc(routed ? a.meta0 + (size_t)e * a.meta_stride : a.smeta0, nm);
+        if constexpr (GATEUP) {
+          rq[1] = make_rsrc(routed ? a.qs1 + (size_t)e * a.qs_stride : a.sqs1, nq);
+          rm[1] = make_rsrc(routed ? a.meta1 + (size_t)e * a.meta_stride : a.smeta1, nm);
+        }
       }
-    }
-    // The planes are in panels of 64 segments (nx_device.hpp): the chunk's
-    // panel grp starts at grp * rows * prq (codes) and grp * rows * prm
-    // (scales), prq and prm a row's bytes in a panel, and holds gsz segments
-    // of each row.  Per-lane parts of the offsets stay in registers; the rest
-    // goes in the scalar offset.  Steps past the run's rows (the
-    // pipeline's tail) and chunks past the row read at OOB.
-    constexpr int SPC = Q80 ? 8 : 4;                               // segments per chunk
-    constexpr int QU = Q2K ? 16 : 32, MU = Q80 ? 2 : Q2K ? 8 : 4;  // plane bytes per segment
-    const uint32_t prq = panel_row_bytes(a.nseg, QU), prm = panel_row_bytes(a.nseg, MU);
-    const int j0 = SPC * (in_row ? c : 0), grp = j0 >> 6, gsz = min(64, a.nseg - (grp << 6));
-    const uint32_t vq = (uint32_t)l16 * prq + (Q80 ? 32u : 16u) * (uint32_t)g;
-    const uint32_t vm = (uint32_t)l16 * prm + (Q2K ? 8u * (uint32_t)g : 0u);
-    const uint32_t sq0 = (uint32_t)grp * (uint32_t)a.rows * prq + (uint32_t)((j0 & 63) * 16);
-    const uint32_t sm0 = (uint32_t)grp * (uint32_t)a.rows * prm + (uint32_t)((j0 & 63) * MU);
-    // step i of the pass from row tile rt: gate/up row tile rt + i / 2 of gate
-    // (i even) or up
-    auto issue = [&](MfvStep<FMT> &w, int rt, int i) {
-      rt += GATEUP ? i >> 1 : i;
-      const int mt = GATEUP ? i & 1 : 0;
-      const bool in = in_row && rt < rt1;  // wave-uniform
-      const uint32_t past = in ? 0u : OOB;
-      const uint32_t sq = in ? sq0 + 16u * rt * prq : 0u, smo = in ? sm0 + 16u * rt * prm : 0u;
+      // The planes are in panels of 64 segments (nx_device.hpp): the chunk's
+      // panel grp starts at grp * rows * prq (codes) and grp * rows * prm
+      // (scales), prq and prm a row's bytes in a panel, and holds gsz segments
+      // of each row.  Per-lane parts of the offsets stay in registers; the rest
+      // goes in the scalar offset.  Steps past the run's rows (the
+      // pipeline's tail) and chunks past the row read at OOB.
+      constexpr int SPC = Q80 ? 8 : 4;                               // segments per chunk
+      constexpr int QU = Q2K ? 16 : 32, MU = Q80 ? 2 : Q2K ? 8 : 4;  // plane bytes per segment
+      const uint32_t prq = panel_row_bytes(a.nseg, QU), prm = panel_row_bytes(a.nseg, MU);
+      const int j0 = SPC * (in_row ? c : 0), grp = j0 >> 6, gsz = min(64, a.nseg - (grp << 6));
+      const uint32_t vq = (uint32_t)l16 * prq + (Q80 ? 32u : 16u) * (uint32_t)g;
+      const uint32_t vm = (uint32_t)l16 * prm + (Q2K ? 8u * (uint32_t)g : 0u);
+      const uint32_t sq0 = (uint32_t)grp * (uint32_t)a.rows * prq + (uint32_t)((j0 & 63) * 16);
+      const uint32_t sm0 = (uint32_t)grp * (uint32_t)a.rows * prm + (uint32_t)((j0 & 63) * MU);
+      // step i of the pass from row tile rt: gate/up row tile rt + i / 2 of gate
+      // (i even) or up
+      auto issue = [&](MfvStep<FMT> &w, int rt, int i) {
+        rt += GATEUP ? i >> 1 : i;
+        const int mt = GATEUP ? i & 1 : 0;
+        const bool in = in_row && rt < rt1;  // wave-uniform
+        const uint32_t past = in ? 0u : OOB;
+        const uint32_t sq = in ? sq0 + 16u * rt * prq : 0u, smo = in ? sm0 + 16u * rt * prm : 0u;
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        // Q8_0: [2 t + h] = half h of block 2 g + t; Q4: half q of segment g
-        const int h = Q80 ? (q & 1) : q, t = Q80 ? (q >> 1) : 0;
-        w.q[q] = __builtin_amdgcn_raw_buffer_load_b128(rq[mt], (int)(vq | past),
-                                                       (int)(sq + (in ? h * 16 * gsz + 16 * t : 0)), 0);
-      }
-      if constexpr (Q2K) {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b64(rm[mt], (int)(vm | past), (int)smo, 0);
-        w.m = u32x4_t{v[0], v[1], 0, 0};
-      } else {
-        w.m = __builtin_amdgcn_raw_buffer_load_b128(rm[mt], (int)(vm | past), (int)smo, 0);
-      }
-    };
-    // the first steps go out ahead of the chain of loads that finds the pairs'
-    // records
-    MfvStep<FMT> ring[MV_STEPS];  // slot i: step i of a pass; D of them live
+        for (int q = 0; q < NQ; ++q) {
+          // Q8_0: [2 t + h] = half h of block 2 g + t; Q4: half q of segment g
+          const int h = Q80 ? (q & 1) : q, t = Q80 ? (q >> 1) : 0;
+          w.q[q] = __builtin_amdgcn_raw_buffer_load_b128(rq[mt], (int)(vq | past),
+                                                         (int)(sq + (in ? h * 16 * gsz + 16 * t : 0)), 0);
+        }
+        if constexpr (Q2K) {
+          const auto v = __builtin_amdgcn_raw_buffer_load_b64(rm[mt], (int)(vm | past), (int)smo, 0);
+          w.m = u32x4_t{v[0], v[1], 0, 0};
+        } else {
+          w.m = __builtin_amdgcn_raw_buffer_load_b128(rm[mt], (int)(vm | past), (int)smo, 0);
+        }
+      };
+      // the first steps go out ahead of the chain of loads that finds the pairs'
+      // records
+      MfvStep<FMT> ring[MV_STEPS];  // slot i: step i of a pass; D of them live
 #pragma unroll
-    for (int i = 0; i < D; ++i) issue(ring[i], rt0, i);
-    __builtin_amdgcn_sched_barrier(0);
+      for (int i = 0; i < D; ++i) issue(ring[i], rt0, i);
+      __builtin_amdgcn_sched_barrier(0);
 
-    // ---- activations: lane's row of the tile (absent pairs take the last
-    // one's, and are not stored)
-    const int m = min(l16, cnt - 1);
-    const int xr = a.perm_token ? (routed ? a.perm_token[pair0 + m] : m0 + m) : pair0 + m;
-    const uint8_t *rec = a.rec + ((size_t)xr * a.nchunk + (in_row ? c : 0)) * REC_BYTES;
-    f16x8 hi[8], lo[8];
+      // ---- activations: lane's row of the tile (absent pairs take the last
+      // one's, and are not stored)
+      const int m = min(l16, cnt - 1);
+      const int xr = a.perm_token ? (routed ? a.perm_token[pair0 + m] : m0 + m) : pair0 + m;
+      const uint8_t *rec = a.rec + ((size_t)xr * a.nchunk + (in_row ? c : 0)) * REC_BYTES;
+      f16x8 hi[8], lo[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      hi[u] = *reinterpret_cast<const f16x8 *>(rec + 128 * u + 16 * g);
-      lo[u] = *reinterpret_cast<const f16x8 *>(rec + 128 * u + 64 + 16 * g);
-    }
-    u32x4_t xm = {0, 0, 0, 0};
-    if constexpr (Q4K) {
-      const uint2 v = *reinterpret_cast<const uint2 *>(rec + REC_XM + 8 * g);
-      xm.x = v.x;
-      xm.y = v.y;
-    } else if constexpr (Q2K) {
-      xm = *reinterpret_cast<const u32x4_t *>(rec + REC_XM + 16 * g);
-    }
-    const float sxl = *reinterpret_cast<const float *>(rec + REC_SX);
-    float sx[4];
+      for (int u = 0; u < 8; ++u) {
+        hi[u] = *reinterpret_cast<const f16x8 *>(rec + 128 * u + 16 * g);
+        lo[u] = *reinterpret_cast<const f16x8 *>(rec + 128 * u + 64 + 16 * g);
+      }
+      u32x4_t xm = {0, 0, 0, 0};
+      if constexpr (Q4K) {
+        const uint2 v = *reinterpret_cast<const uint2 *>(rec + REC_XM + 8 * g);
+        xm.x = v.x;
+        xm.y = v.y;
+      } else if constexpr (Q2K) {
+        xm = *reinterpret_cast<const u32x4_t *>(rec + REC_XM + 16 * g);
+      }
+      const float sxl = *reinterpret_cast<const float *>(rec + REC_SX);
+      float sx[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) sx[k] = in_row ? __shfl(sxl, 4 * g + k, 64) : 0.f;
+      for (int k = 0; k < 4; ++k) sx[k] = in_row ? __shfl(sxl, 4 * g + k, 64) : 0.f;
 
-    float *out = a.out + (size_t)slice * a.out_split + (size_t)(pair0 + 4 * g) * a.out_stride + l16;
+      float *out = a.out + (size_t)slice * a.out_split + (size_t)(pair0 + 4 * g) * a.out_stride + l16;
 #pragma clang loop unroll(disable)
-    for (int rt = rt0; rt < rt1; rt += RT) {
+      for (int rt = rt0; rt < rt1; rt += RT) {
 #pragma unroll
-      for (int i = 0; i < MV_STEPS; ++i) {
-        MfvStep<FMT> &w = ring[i];
+        for (int i = 0; i < MV_STEPS; ++i) {
+          MfvStep<FMT> &w = ring[i];
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) asm volatile("" : "+v"(w.q[q]));
-        asm volatile("" : "+v"(w.m));
-        f32x4 y = f32x4{0.f, 0.f, 0.f, 0.f}, res;
-        // MFMA u of operand b, both halves
-        auto mfma = [&](int u, f16x8 b, f32x4 y4) {
-          y4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[u], b, y4, 0, 0, 0);
-          return __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[u], b, y4, 0, 0, 0);
-        };
-        if constexpr (BLK) {
-          // the loads give lane group g blocks 2 g and 2 g + 1; transposed
-          // across the lane groups, it holds its 8 weights of every block
-          constexpr int NW = Q80 ? 2 : 1;
-          uint32_t cq[2][NW][4];
+          for (int q = 0; q < NQ; ++q) asm volatile("" : "+v"(w.q[q]));
+          asm volatile("" : "+v"(w.m));
+          f32x4 y = f32x4{0.f, 0.f, 0.f, 0.f}, res;
+          // MFMA u of operand b, both halves
+          auto mfma = [&](int u, f16x8 b, f32x4 y4) {
+            y4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[u], b, y4, 0, 0, 0);
+            return __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[u], b, y4, 0, 0, 0);
+          };
+          if constexpr (BLK) {
+            // the loads give lane group g blocks 2 g and 2 g + 1; transposed
+            // across the lane groups, it holds its 8 weights of every block
+            constexpr int NW = Q80 ? 2 : 1;
+            uint32_t cq[2][NW][4];
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            if constexpr (Q80) {
-              const u32x4_t q0 = w.q[2 * h], q1 = w.q[2 * h + 1];
-              cq[h][0][0] = q0.x, cq[h][0][1] = q0.z, cq[h][0][2] = q1.x, cq[h][0][3] = q1.z;
-              cq[h][NW - 1][0] = q0.y, cq[h][NW - 1][1] = q0.w, cq[h][NW - 1][2] = q1.y, cq[h][NW - 1][3] = q1.w;
-            } else {
-              const u32x4_t q0 = w.q[h];
-              cq[h][0][0] = q0.x, cq[h][0][1] = q0.y, cq[h][0][2] = q0.z, cq[h][0][3] = q0.w;
+            for (int h = 0; h < 2; ++h) {
+              if constexpr (Q80) {
+                const u32x4_t q0 = w.q[2 * h], q1 = w.q[2 * h + 1];
+                cq[h][0][0] = q0.x, cq[h][0][1] = q0.z, cq[h][0][2] = q1.x, cq[h][0][3] = q1.z;
+                cq[h][NW - 1][0] = q0.y, cq[h][NW - 1][1] = q0.w, cq[h][NW - 1][2] = q1.y, cq[h][NW - 1][3] = q1.w;
+              } else {
+                const u32x4_t q0 = w.q[h];
+                cq[h][0][0] = q0.x, cq[h][0][1] = q0.y, cq[h][0][2] = q0.z, cq[h][0][3] = q0.w;
+              }
+#pragma unroll
+              for (int v = 0; v < NW; ++v) transpose_groups(cq[h][v]);
+            }
+            // codes at 2^-9
+            const f16x2 s1 = {32768.0f16, 32768.0f16}, s16 = {2048.0f16, 2048.0f16};
+            const f16x2 off = {-0x1p-6f16, -0x1p-6f16};
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+              const f16x8 bq = Q80 ? operand8(cq[b & 1][0][b >> 1], cq[b & 1][NW - 1][b >> 1])
+                                   : operand4(cq[b & 1][0][b >> 1], s1, s16, off);
+              const uint32_t dw = w.m[b >> 1];
+              const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(b & 1 ? dw >> 16 : dw & 0xFFFFu));
+              const f32x4 z = mfma(b, bq, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+              for (int k = 0; k < 4; ++k) y[k] = fmaf(d, z[k], y[k]);
+              // one step's operands live at a time: left free, the compiler
+              // forms every step's operands first and spills
+              asm volatile("" : "+v"(y));
             }
 #pragma unroll
-            for (int v = 0; v < NW; ++v) transpose_groups(cq[h][v]);
-          }
-          // codes at 2^-9
-          const f16x2 s1 = {32768.0f16, 32768.0f16}, s16 = {2048.0f16, 2048.0f16};
-          const f16x2 off = {-0x1p-6f16, -0x1p-6f16};
+            for (int k = 0; k < 4; ++k) res[k] = sx[k] * 512.0f * y[k];
+          } else {
+            // scales into the operands, sc 2^10 and sc 2^6 (2^-14 with the codes'
+            // 2^-24); mins for their own MFMA
+            constexpr int NV = Q2K ? 4 : 2;
+            uint32_t scv[NV], mnv[NV];
+            if constexpr (Q2K) {
 #pragma unroll
-          for (int b = 0; b < 8; ++b) {
-            const f16x8 bq = Q80 ? operand8(cq[b & 1][0][b >> 1], cq[b & 1][NW - 1][b >> 1])
-                                 : operand4(cq[b & 1][0][b >> 1], s1, s16, off);
-            const uint32_t dw = w.m[b >> 1];
-            const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(b & 1 ? dw >> 16 : dw & 0xFFFFu));
-            const f32x4 z = mfma(b, bq, f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int k = 0; k < 4; ++k) y[k] = fmaf(d, z[k], y[k]);
-            // one step's operands live at a time: left free, the compiler
-            // forms every step's operands first and spills
-            asm volatile("" : "+v"(y));
-          }
-#pragma unroll
-          for (int k = 0; k < 4; ++k) res[k] = sx[k] * 512.0f * y[k];
-        } else {
-          // scales into the operands, sc 2^10 and sc 2^6 (2^-14 with the codes'
-          // 2^-24); mins for their own MFMA
-          constexpr int NV = Q2K ? 4 : 2;
-          uint32_t scv[NV], mnv[NV];
-          if constexpr (Q2K) {
+              for (int v = 0; v < NV; ++v) {
+                scv[v] = (w.m.y >> (8 * v)) & 15;
+                mnv[v] = (w.m.y >> (8 * v + 4)) & 15;
+              }
+            } else {
+              // get_scale_min_k4 (src/quant/mod.rs:1163-1170) of sub-blocks g, g + 4
+              const uint32_t p03 = w.m.y, p47 = w.m.z, p8b = w.m.w;
+              scv[0] = (p03 >> (8 * g)) & 63;
+              mnv[0] = (p47 >> (8 * g)) & 63;
+              scv[NV - 1] = ((p8b >> (8 * g)) & 15) | (((p03 >> (8 * g + 6)) & 3) << 4);
+              mnv[NV - 1] = ((p8b >> (8 * g + 4)) & 15) | (((p47 >> (8 * g + 6)) & 3) << 4);
+            }
+            f16x2 s1[NV], s16[NV], off[NV];
+            _Float16 mn[NV];
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
-              scv[v] = (w.m.y >> (8 * v)) & 15;
-              mnv[v] = (w.m.y >> (8 * v + 4)) & 15;
+              const _Float16 f = (_Float16)(float)(scv[v] << 10);
+              s1[v] = f16x2{f, f};
+              s16[v] = s1[v] * f16x2{0.0625f16, 0.0625f16};
+              off[v] = s16[v] * f16x2{-0x1p-17f16, -0x1p-17f16};  // -8 sc 2^-14
+              mn[v] = (_Float16)(float)mnv[v];
             }
-          } else {
-            // get_scale_min_k4 (src/quant/mod.rs:1163-1170) of sub-blocks g, g + 4
-            const uint32_t p03 = w.m.y, p47 = w.m.z, p8b = w.m.w;
-            scv[0] = (p03 >> (8 * g)) & 63;
-            mnv[0] = (p47 >> (8 * g)) & 63;
-            scv[NV - 1] = ((p8b >> (8 * g)) & 15) | (((p03 >> (8 * g + 6)) & 3) << 4);
-            mnv[NV - 1] = ((p8b >> (8 * g + 4)) & 15) | (((p47 >> (8 * g + 6)) & 3) << 4);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+              f16x8 b;
+              if constexpr (Q2K)  // the 2-bit codes of half u / 4 widened to nibbles (no offset)
+                b = operand4u((w.q[0][u & 3] >> (2 * (u >> 2))) & 0x33333333u, s1[u >> 1], s16[u >> 1]);
+              else
+                b = operand4(w.q[(u >> 2) % NQ][u & 3], s1[(u >> 2) % NV], s16[(u >> 2) % NV], off[(u >> 2) % NV]);
+              y = mfma(u, b, y);
+              asm volatile("" : "+v"(y));  // as above
+            }
+            const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(w.m.x & 0xFFFF));
+            const float dmin = (float)__builtin_bit_cast(_Float16, (uint16_t)(w.m.x >> 16));
+            const float dd = d * 16384.0f, dm = dmin * 64.0f;  // X enters 2^-6
+            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+            f32x4 rest;  // what the offsets and mins add
+            if constexpr (Q2K) {
+              const f32x4 ym = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                  __builtin_bit_cast(f16x8, xm), f16x8{mn[0], mn[0], mn[1], mn[1], mn[NV - 2], mn[NV - 2], mn[NV - 1], mn[NV - 1]},
+                  zero, 0, 0, 0);
+#pragma unroll
+              for (int k = 0; k < 4; ++k) rest[k] = -dm * ym[k];
+            } else {
+              // 8 sc X at the codes' 2^-14 (X enters 2^-6): sc 2^-5; and m.  On
+              // accumulators of their own: the result of an MFMA of one shape, taken
+              // as another shape's accumulator, is read before it is complete unless
+              // enough instructions lie between, and the compiler (ROCm 7.2) puts no
+              // wait there.  16x16x32 and 16x16x16 back to back on one accumulator
+              // lose the first in two of the four registers.
+              const f16x4 xa = __builtin_bit_cast(f16x4, uint2{xm.x, xm.y});
+              const _Float16 k15 = (_Float16)0x1p-15f;
+              const _Float16 b0 = s1[0][0] * k15, b1 = s1[NV - 1][0] * k15;
+              const f32x4 yx = __builtin_amdgcn_mfma_f32_16x16x16f16(xa, f16x4{b0, b0, b1, b1}, zero, 0, 0, 0);
+              const f32x4 ym = __builtin_amdgcn_mfma_f32_16x16x16f16(
+                  xa, f16x4{mn[0], mn[0], mn[NV - 1], mn[NV - 1]}, zero, 0, 0, 0);
+#pragma unroll
+              for (int k = 0; k < 4; ++k) rest[k] = fmaf(dd, yx[k], -dm * ym[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) res[k] = sx[k] * fmaf(dd, y[k], rest[k]);
           }
-          f16x2 s1[NV], s16[NV], off[NV];
-          _Float16 mn[NV];
-#pragma unroll
-          for (int v = 0; v < NV; ++v) {
-            const _Float16 f = (_Float16)(float)(scv[v] << 10);
-            s1[v] = f16x2{f, f};
-            s16[v] = s1[v] * f16x2{0.0625f16, 0.0625f16};
-            off[v] = s16[v] * f16x2{-0x1p-17f16, -0x1p-17f16};  // -8 sc 2^-14
-            mn[v] = (_Float16)(float)mnv[v];
-          }
-#pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            f16x8 b;
-            if constexpr (Q2K)  // the 2-bit codes of half u / 4 widened to nibbles (no offset)
-              b = operand4u((w.q[0][u & 3] >> (2 * (u >> 2))) & 0x33333333u, s1[u >> 1], s16[u >> 1]);
-            else
-              b = operand4(w.q[(u >> 2) % NQ][u & 3], s1[(u >> 2) % NV], s16[(u >> 2) % NV], off[(u >> 2) % NV]);
-            y = mfma(u, b, y);
-            asm volatile("" : "+v"(y));  // as above
-          }
-          const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(w.m.x & 0xFFFF));
-          const float dmin = (float)__builtin_bit_cast(_Float16, (uint16_t)(w.m.x >> 16));
-          const float dd = d * 16384.0f, dm = dmin * 64.0f;  // X enters 2^-6
-          const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-          f32x4 rest;  // what the offsets and mins add
-          if constexpr (Q2K) {
-            const f32x4 ym = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                __builtin_bit_cast(f16x8, xm), f16x8{mn[0], mn[0], mn[1], mn[1], mn[NV - 2], mn[NV - 2], mn[NV - 1], mn[NV - 1]},
-                zero, 0, 0, 0);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) rest[k] = -dm * ym[k];
-          } else {
-            // 8 sc X at the codes' 2^-14 (X enters 2^-6): sc 2^-5; and m.  On
-            // accumulators of their own: the result of an MFMA of one shape, taken
-            // as another shape's accumulator, is read before it is complete unless
-            // enough instructions lie between, and the compiler (ROCm 7.2) puts no
-            // wait there.  16x16x32 and 16x16x16 back to back on one accumulator
-            // lose the first in two of the four registers.
-            const f16x4 xa = __builtin_bit_cast(f16x4, uint2{xm.x, xm.y});
-            const _Float16 k15 = (_Float16)0x1p-15f;
-            const _Float16 b0 = s1[0][0] * k15, b1 = s1[NV - 1][0] * k15;
-            const f32x4 yx = __builtin_amdgcn_mfma_f32_16x16x16f16(xa, f16x4{b0, b0, b1, b1}, zero, 0, 0, 0);
-            const f32x4 ym = __builtin_amdgcn_mfma_f32_16x16x16f16(
-                xa, f16x4{mn[0], mn[0], mn[NV - 1], mn[NV - 1]}, zero, 0, 0, 0);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) rest[k] = fmaf(dd, yx[k], -dm * ym[k]);
-          }
-#pragma unroll
-          for (int k = 0; k < 4; ++k) res[k] = sx[k] * fmaf(dd, y[k], rest[k]);
+          __builtin_amdgcn_sched_barrier(0);
+          issue(ring[(i + D) % MV_STEPS], i + D < MV_STEPS ? rt : rt + RT, (i + D) % MV_STEPS);
+          __builtin_amdgcn_sched_barrier(0);
+          red[buf + (wave * MV_STEPS + i) * 64 + lane] = res;
         }
-        __builtin_amdgcn_sched_barrier(0);
-        issue(ring[(i + D) % MV_STEPS], i + D < MV_STEPS ? rt : rt + RT, (i + D) % MV_STEPS);
-        __builtin_amdgcn_sched_barrier(0);
-        red[buf + (wave * MV_STEPS + i) * 64 + lane] = res;
-      }
-      // The slice's sums: every pass the waves leave their chunks' results in one
-      // of two buffers, and wave w adds those of steps w, w + ks, ... in chunk
-      // order.  One barrier per pass: a buffer is written again only after the
-      // next pass's barrier.
-      __syncthreads();
-      for (int t = wave; t < MV_STEPS; t += a.ks) {
-        const f32x4 *r = red + buf + t * 64 + lane;
-        f32x4 sum = *r;
-        for (int v = 1; v < a.ks; ++v) {
-          r += MV_STEPS * 64;
+        // The slice's sums: every pass the waves leave their chunks' results in one
+        // of two buffers, and wave w adds those of steps w, w + ks, ... in chunk
+        // order.  One barrier per pass: a buffer is written again only after the
+        // next pass's barrier.
+        __syncthreads();
+        for (int t = wave; t < MV_STEPS; t += a.ks) {
+          const f32x4 *r = red + buf + t * 64 + lane;
+          f32x4 sum = *r;
+          for (int v = 1; v < a.ks; ++v) {
+            r += MV_STEPS * 64;
 #pragma unroll
-          for (int k = 0; k < 4; ++k) sum[k] += (*r)[k];
+            for (int k = 0; k < 4; ++k) sum[k] += (*r)[k];
+          }
+          // lane holds row (lane % 16), pairs 4g .. 4g+3
+          float *o = out + (GATEUP ? 16 * (rt + (t >> 1)) + (t & 1) * a.rows : 16 * (rt + t));
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            if (4 * g + k < cnt) o[(size_t)k * a.out_stride] = sum[k];
         }
-        // lane holds row (lane % 16), pairs 4g .. 4g+3
-        float *o = out + (GATEUP ? 16 * (rt + (t >> 1)) + (t & 1) * a.rows : 16 * (rt + t));
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          if (4 * g + k < cnt) o[(size_t)k * a.out_stride] = sum[k];
+        buf ^= a.ks * MV_STEPS * 64;
       }
-      buf ^= a.ks * MV_STEPS * 64;
     }
   }
 }

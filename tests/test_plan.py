@@ -19,7 +19,7 @@ pytestmark = pytest.mark.skipif(GXX is None, reason="no host C++ compiler")
 def run(tmp_path, body):
     """Compiles `body` as main()'s statements over the header and runs it."""
     src, exe = tmp_path / "check.cpp", tmp_path / "check"
-    src.write_text('#include <cstdio>\n#include "nx_plan.hpp"\nusing namespace nx;\n'
+    src.write_text('#include <cstdio>\n#include <vector>\n#include "nx_plan.hpp"\nusing namespace nx;\n'
                    "int main() {\n  int bad = 0;\n" + body + "\n  return bad ? 1 : 0;\n}\n")
     r = subprocess.run([GXX, "-std=c++17", "-O1", "-Wall", "-Werror", f"-I{CSRC}", str(src), "-o", str(exe)],
                        capture_output=True, text=True)
@@ -111,24 +111,27 @@ def test_split_workspace(tmp_path):
 
 
 def test_split_runs_cover_the_line_once(tmp_path):
-    """The workgroups' runs of the split kernel follow each other over the whole
-    line, each unit once, and none is longer than an equal share and two passes."""
+    """The workgroups' runs of the split kernel cover the whole line, each unit
+    once; whole segments but in the last round, where none is longer than an
+    equal share and two passes."""
     run(tmp_path, r"""
   for (int nb : {256, 512, 304, 1})
-    for (int nseg = 0; nseg <= 700; nseg += nseg < 40 ? 1 : 13)
+    for (int nseg = 0; nseg <= 1100; nseg += nseg < 40 ? 1 : 13)
       for (int npass : {2, 4, 5, 8, 20, 32, 64, 112, 448}) {
-        long at = 0, most = 0;
-        for (int b = 0; b < nb; ++b) {
-          const MfvRun r = mfv_run(b, nb, nseg, npass);
-          if (r.u0 != at || r.u1 < r.u0) ++bad;
-          at = r.u1;
-          most = std::max(most, r.u1 - r.u0);
-        }
-        const long work = (long)nseg * npass;
-        if (at != work || most > (work + nb - 1) / nb + 2) {
-          std::printf("%d workgroups, %d segments of %d: %ld of %ld, at most %ld\n", nb, nseg, npass, at, work, most);
-          ++bad;
-        }
+        std::vector<int> seen((size_t)nseg * npass);
+        for (int first = 0, left = nseg; left > 0; first += nb, left -= nb)
+          for (int b = 0; b < nb; ++b) {
+            const MfvRun r = mfv_run(b, nb, left, npass);
+            const long share = ((long)left * npass + nb - 1) / nb;
+            if (r.u1 < r.u0 || r.u1 - r.u0 > (left >= nb ? npass : share + 2)) ++bad;
+            for (int u = r.u0; u < r.u1; ++u) ++seen.at((size_t)(first + r.seg0) * npass + u);
+          }
+        for (int v : seen)
+          if (v != 1) {
+            std::printf("%d workgroups, %d segments of %d\n", nb, nseg, npass);
+            ++bad;
+            break;
+          }
       }
 """)
 
