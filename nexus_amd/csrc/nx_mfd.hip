@@ -41,7 +41,7 @@
 // the time, waves waiting 27% of theirs for memory or a barrier and 36% for
 // issue; 32000 x 4096 Q8_0, 13 tokens: 38%, 7%, 32% and 43%.  Measured against
 // the GEMV (us): 4096 x 4096 Q4_K, 5 tokens 12.8 -> 9.2, 64 tokens 112 -> 17.0,
-// 509 tokens 874 -> 54-58; 32000 x 4096 Q8_0, 13 tokens 159 -> 44.5 (3.2 TB/s of
+// 509 tokens 874 -> 54-64; 32000 x 4096 Q8_0, 13 tokens 159 -> 44.5 (3.2 TB/s of
 // weights).  Error against
 // 64 bits 2.1e-7 (Q4_K) and 1.1e-7 (Q4_0, Q8_0), the GEMV's 3.0e-7 and 2.7e-7.
 #include "nx_internal.hpp"

@@ -44,8 +44,8 @@
 // tokens, gate/up (529 MB) 127 us, of which the loads alone take 123 and the
 // arithmetic alone 99.  Against workgroups of 256 rows that staged their
 // activations in LDS and walked a slice of 4 chunks (us, layer): Mixtral 32
-// tokens 246 -> 212, DeepSeek 27 tokens 1049 -> 836, Qwen3 61 tokens 118.5 ->
-// 108.9; error against 64 bits 9.3e-7 -> 3.8e-7 (Q4_K), 7.8e-5 -> 2.1e-7 (Q4_0,
+// tokens 250 -> 214, DeepSeek 27 tokens 1071 -> 831, Qwen3 61 tokens 119.8 ->
+// 109.2; error against 64 bits 9.3e-7 -> 3.8e-7 (Q4_K), 7.8e-5 -> 2.1e-7 (Q4_0,
 // whose codes were fp16 subnormals).  A wave per 64 rows that walked the chunks
 // itself read each line's halves a chunk apart, too late for the L2: 370 us.
 #include "nx_internal.hpp"

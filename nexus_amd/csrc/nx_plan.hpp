@@ -144,11 +144,11 @@ inline int auto_path(const MoeShape &s, int T, int k, bool aligned, size_t scrat
     // A shared expert sees every token: the GEMV walks it a token pair at
     // a time, the split-activation path 16 tokens at a time.  Measured
     // (DeepSeek shapes, us, GEMV / split / grouped GEMM): Q4_K 2 tokens 107 /
-    // 117 / 238, 4: 263 / 183 / 283, 8: 874 / 331 / 580, 27: - / 867 / 1262,
-    // 128: - / 1562 / 2018, 256 (8 per routed expert): - / 1794 / 2122, 384
-    // (12): - / 1952 / 2151; Q4_0 2: 98 / 123 / 235, 4: 237 / 204 / 364, 27: - /
-    // 842 / 1241, 384: - / 1937 / 2104; Q8_0 4: 315 / 323 / 450, 8: 847 / 557 /
-    // 676, 128: - / 2425 / 2554, 256: - / 2772 / 2702.
+    // 117 / 238, 4: 263 / 183 / 283, 8: 874 / 331 / 580, 27: - / 814 / 1223,
+    // 128: - / 1543 / 2046, 256 (8 per routed expert): - / 1702 / 2141, 384
+    // (12): - / 1853 / 2195; Q4_0 2: 98 / 123 / 235, 4: 237 / 200 / 293, 27: - /
+    // 839 / 1187, 384: - / 1870 / 2147; Q8_0 4: 315 / 313 / 370, 8: 847 / 529 /
+    // 650, 128: - / 2398 / 2559, 256: - / 2696 / 2700, 384: - / 2934 / 2772.
     if (tpe >= (large && !q8 ? 12.0 : 8.0)) return NX_PATH_MFMA_BF16;
     return T >= (q8 ? 6 : 4) ? NX_PATH_MFMA_SPLIT : NX_PATH_GEMV;
   }
